@@ -96,6 +96,23 @@ constexpr GemmTile kGemmTiles[] = {{128, 2, 4, 1}, {128, 1, 4, 1}, {128, 3, 4, 1
                                    {64, 1, 4, 3},  {32, 1, 8, 2},  {64, 1, 8, 2}};
 constexpr int kNumGemmTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
+// Fragment GEMM tiles (gemm_frag.hip): WR x WC waves of WA x WB 32 x 32 blocks each, in the order of
+// BRIK_FRAG_TILES: 192 x 256, 128 x 256, 128 x 128, 64 x 128. `slice_us`: time of a 16-k slice per round of
+// CUs, measured on the product alone. Swept at (M, K, N) = (4096, 9728, 2560), (2048 and 1024, 2560, 9728),
+// (777, 2560, 4096), (512, 2560, 9728), (4096, 2560, 320): each of the four is the fastest of 18 tiles
+// (64-256 rows, 128-256 columns, 4 and 8 waves) on one of them, 174, 98, 53, 21.7, 29.9 and 12.4 us.
+struct FragTile {
+    int wr, wc, wa, wb;
+    double slice_us;
+    int bm() const { return 32 * wr * wa; }
+    int bn() const { return 32 * wc * wb; }
+    unsigned threads() const { return 64u * (unsigned)(wr * wc); }
+};
+constexpr FragTile kFragTiles[] = {{2, 4, 3, 2, 0.29}, {1, 8, 4, 1, 0.165}, {1, 4, 4, 1, 0.115}, {1, 4, 2, 1, 0.068}};
+constexpr int kNumFragTiles = sizeof(kFragTiles) / sizeof(kFragTiles[0]);
+// dequantized weight panels held at a time: wider matrices run in column slabs of this many bytes
+constexpr size_t kFragSlabBytes = 128u << 20;
+
 constexpr unsigned kCUs = 256;                 // MI355X compute units
 constexpr long kGemmKPad = 256;                // staged activation rows are padded to this many halves
 constexpr size_t kGemvMaxLds = 64 * 1024;      // dynamic LDS budget of one GEMV block
@@ -190,6 +207,8 @@ struct brik_ctx {
     hipFunction_t gemmg_adapt[2] = {};           // brik_gemmg_q4_64a (4 waves), brik_gemmg_q4_64aw8 (8 waves)
     hipFunction_t gemm_f16[kNumGemmTiles] = {};   // f16-weight tiles (TN = 1, PF = 1 only; others null)
     hipFunction_t gemm_sk[3][3] = {};      // split-K few-row kernels, KSL = 2, 4, 8
+    hipFunction_t frag_prep[3] = {};             // brik_frag_prep_<fmt>
+    hipFunction_t gemm_frag[kNumFragTiles] = {};  // brik_gemm_frag_<tile>
     hipStream_t stream = nullptr;
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
     int opt_path = 0;
@@ -209,6 +228,8 @@ struct brik_ctx {
     size_t cws_bytes = 0;
     void* pws = nullptr;   // split-K partial tiles [slice][row][column] f32 (grow-only)
     size_t pws_bytes = 0;
+    void* fws = nullptr;   // fragment GEMM: the dequantized f16 weight panels of one column slab (grow-only)
+    size_t fws_bytes = 0;
 
     // pinned staging ring of brik_h2d_async (allocated on first use): uploads in flight as
     // {offset, bytes, event} in issue order; events are recycled through a free list
@@ -424,6 +445,9 @@ size_t gemm_stage_bytes(long rows, long K, long& Kp)
     return (size_t)rows * Kp * 2 + 4 * (size_t)rows;
 }
 
+// Bytes of `rows` rows as fragment panels (32 rows, K padded to 128) and their row scales.
+size_t frag_stage_bytes(long rows, long K) { return (size_t)((rows + 31) / 32) * ((K + 127) / 128 * 8) * 1024 + 4 * (size_t)rows; }
+
 // Workspace for `rows` staged f16 activation rows of K (padded to Kp) and their row scales.
 int gemm_stage_ws(brik_ctx* c, int rows, int K, long& Kp, uint16_t*& xh, float*& rscale,
                   const Scratch* fixed = nullptr)
@@ -433,7 +457,9 @@ int gemm_stage_ws(brik_ctx* c, int rows, int K, long& Kp, uint16_t*& xh, float*&
     if (xbytes >= (1ull << 31))
         return fail(c, BRIK_EINVAL, "matmul: %d rows x K=%d exceed the 2 GiB staged-activation limit", rows, K);
     void* p = nullptr;
-    HIP_TRY_RC(take_scratch(c, fixed, c->ws, c->ws_bytes, bytes, p));
+    // when the workspace has to grow, by enough for the fragment GEMM's whole panels of 32 rows too
+    const size_t want = !fixed && c->ws_bytes < bytes ? std::max(bytes, frag_stage_bytes(rows, K)) : bytes;
+    HIP_TRY_RC(take_scratch(c, fixed, c->ws, c->ws_bytes, want, p));
     xh = static_cast<uint16_t*>(p);
     rscale = reinterpret_cast<float*>(static_cast<char*>(p) + xbytes);
     return BRIK_OK;
@@ -622,6 +648,121 @@ int gemm_run(brik_ctx* c, Fmt f, const uint16_t* xh, const float* rscale, const 
     return launch_fn(c, fn, blocks, 1, gt.threads(), 0, args);
 }
 
+// Fragment GEMM (gemm_frag.hip): x staged and W dequantized once into MFMA fragment order by one launch,
+// then an f16 GEMM on the fragments; the bits of the tiled GEMM.
+struct FragShape {
+    long S, RB, CB;             // fragments per panel (K padded to 128), panels of x and of W
+    long slab;                  // W panels per column slab
+    size_t xbytes, wbytes;      // workspaces: x fragments and row scales, one slab of W fragments
+};
+
+FragShape frag_shape(long M, long K, long N)
+{
+    FragShape s;
+    s.S = (K + 127) / 128 * 8;
+    s.RB = (M + 31) / 32;
+    s.CB = (N + 31) / 32;
+    s.slab = std::max(8L, (long)(kFragSlabBytes / ((size_t)s.S * 1024)) / 8 * 8);
+    s.xbytes = frag_stage_bytes(M, K);
+    s.wbytes = (size_t)std::min(s.slab, s.CB) * s.S * 1024;
+    return s;
+}
+
+// The tile of fewest rounds of CUs x time per slice.
+int frag_tile(long M, long N)
+{
+    int best = 0;
+    double best_us = 0;
+    for (int t = 0; t < kNumFragTiles; ++t) {
+        const FragTile& g = kFragTiles[t];
+        const double us = g.slice_us * std::ceil((double)gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()) / kCUs);
+        if (t == 0 || us < best_us) {
+            best = t;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+// Whether a dense GEMM dequantizes W ahead of the product: where a model of both sides, fitted on calls of
+// 256-4096 rows (135 points; K 256-9728, N 336-16162, q4 / q8 / q3, weights from the last-level cache),
+// puts the fragment GEMM at least 7 % ahead. Fragment: two launches and the ends of the product 10.2 us,
+// the bytes of the staging (x read and written, W read and written as f16) and of y at 6.2 TB/s, then the
+// slices. Tiled: 6.7 us, x and y at 4.3 TB/s, then rounds of blocks x K steps of 128, each by tile and format.
+// Measured (us per call, tiled -> fragment): q4 K = 9728, N = 2560: M = 1024 90 -> 84, 2048 157 -> 144,
+// 4096 299 -> 238; q3 K = 2560, N = 9728: M = 512 51 -> 48, 1024 90 -> 72, 4096 282 -> 219; below that the
+// staging costs more than it saves (q4 K = 2560, N = 9728, M = 512: 41 against 47).
+bool use_frag(brik_ctx* c, Fmt f, long M, long K, long N)
+{
+    // a captured call keeps the tiled GEMM (the same bits), so that no graph holds the W panels' address;
+    // and the row staging must fit where the tiled GEMM's would have, so that no workspace grows that
+    // would not have grown
+    if (c->opt_tile > 0 || c->graph_capturing || K > 65536) return false;
+    const FragShape s = frag_shape(M, K, N);
+    long Kp;
+    if (s.xbytes >= (1ull << 31) || (c->ws_bytes < s.xbytes && c->ws_bytes >= gemm_stage_bytes(M, K, Kp))) return false;
+    constexpr double kSliceUs[kNumFragTiles] = {0.28, 0.178, 0.086, 0.056};   // per round, as fitted
+    const double mk = (double)M * K, nk = (double)N * K, mn = (double)M * N;
+    const double wb = f == F_Q4 ? 0.625 : f == F_Q8 ? 1.0625 : 0.5;
+    const int ft = frag_tile(M, std::min<long>(N, 32 * s.slab));
+    const double slabs = std::ceil((double)s.CB / s.slab);
+    const double frounds = std::ceil((double)gemm_tiles(M, kFragTiles[ft].bm()) * gemm_tiles(N, kFragTiles[ft].bn()) / kCUs);
+    const double frag_us = 10.2 * slabs + (6 * mk + (2 + wb) * nk + 4 * mn) / 6.2e6 + s.S * frounds * kSliceUs[ft];
+    const GemmTile& g = kGemmTiles[gemm_tile(c, M, N, K, 0)];
+    const double rounds = std::ceil((double)gemm_tiles(M, g.bm) * gemm_tiles(N, g.bn()) / kCUs);
+    const double area = (double)g.bm * g.bn() / 32768;
+    const double step = (g.bn() <= 128 ? 0.48 + 0.0038 * g.bm : (0.74 + 0.007 * g.bm) * g.bn() / 256) +
+                        area * (f == F_Q3 ? 0.45 : f == F_Q8 ? 0.13 : 0);
+    const double tiled_us = 6.7 + (6 * mk + 4 * mn) / 4.3e6 + rounds * ((K + 255) / 256 * 2) * step;
+    return frag_us < 0.93 * tiled_us;
+}
+
+// Returns BRIK_OK with `done` false when the workspaces could not be had (the tiled GEMM needs less).
+int gemm_frag(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, const void* sc, const void* mn,
+              float* y, int M, int K, int N, bool& done)
+{
+    const FragShape s = frag_shape(M, K, N);
+    done = false;
+    if (ensure_buf(c, c->ws, c->ws_bytes, s.xbytes) != BRIK_OK) return BRIK_OK;
+    if (c->fws_bytes < s.wbytes) {
+        // no graph holds this buffer (use_frag), so unlike the others its growth leaves recorded graphs valid
+        if (c->fws) {
+            HIP_TRY(c, hipStreamSynchronize(c->stream));
+            HIP_TRY(c, hipFree(c->fws));
+            c->fws = nullptr;
+            c->fws_bytes = 0;
+        }
+        if (hipMalloc(&c->fws, s.wbytes) != hipSuccess) {
+            (void)hipGetLastError();
+            c->fws = nullptr;
+            return BRIK_OK;
+        }
+        c->fws_bytes = s.wbytes;
+    }
+    done = true;
+    c->last_path = BRIK_PATH_TILED;
+    uint16_t* xf = static_cast<uint16_t*>(c->ws);
+    float* rscale = reinterpret_cast<float*>(static_cast<char*>(c->ws) + (size_t)s.RB * s.S * 1024);
+    uint16_t* wf = static_cast<uint16_t*>(c->fws);
+    int S = (int)s.S;
+    for (long cb0 = 0; cb0 < s.CB; cb0 += s.slab) {
+        int n0 = (int)(32 * cb0), CB = (int)std::min(s.slab, s.CB - cb0), Ns = (int)std::min<long>(32L * CB, N - n0);
+        // the first slab's launch also stages the rows: 8 (or 4, long rows) per block
+        const int rpb = K <= BRIK_FRAG_ROWS8_MAX_K ? 8 : 4;
+        int xblocks = cb0 == 0 ? (M + rpb - 1) / rpb : 0;
+        const unsigned wblocks = (unsigned)(((long)CB * (S / 8) + 15) / 16);
+        void* pargs[] = {&x, &xf, &rscale, &p0, &p1, &sc, &mn, &wf, &M, &K, &n0, &N, &CB, &S, &xblocks};
+        HIP_TRY_RC(launch_fn(c, c->frag_prep[fmt_index(f)], (unsigned)xblocks + wblocks, 1, 1024, 0, pargs));
+        const int t = frag_tile(M, Ns);
+        const FragTile& g = kFragTiles[t];
+        float* ys = y + n0;
+        void* args[] = {&xf, &rscale, &wf, &ys, &M, &Ns, &N, &S};
+        HIP_TRY_RC(launch_fn(c, c->gemm_frag[t], gemm_tiles(M, g.bm()) * gemm_tiles(Ns, g.bn()), 1, g.threads(), 0,
+                             args));
+    }
+    return BRIK_OK;
+}
+
 // MFMA GEMM over `rows` activation rows: stage x as scaled f16 rows in the workspace, then run the
 // tile kernel.
 int gemm(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, const void* sc, const void* mn,
@@ -640,6 +781,11 @@ int gemm(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, con
         if (need > fixed->bytes)
             return fail(c, BRIK_EINVAL, "no-allocation call: needs %zu bytes of scratch (staged rows and split-K "
                         "partial tiles), the fixed buffer holds %zu", need, fixed->bytes);
+    }
+    if (!row_off && !fixed && !use_splitk(c, f, rows, K, N, E) && use_frag(c, f, rows, K, N)) {
+        bool done = false;
+        HIP_TRY_RC(gemm_frag(c, f, x, p0, p1, sc, mn, y, rows, K, N, done));
+        if (done) return BRIK_OK;
     }
     long Kp;
     uint16_t* xh;
@@ -1076,6 +1222,17 @@ int brik_create(int device, brik_ctx** out)
                 max_threads < (int)kGemmTiles[t].threads())
                 return bail(BRIK_EMODULE);
         }
+    for (int f = 0; f < 3; ++f) {
+        char name[64];
+        snprintf(name, sizeof name, "brik_frag_prep_%s", kFmtNames[f]);
+        if (hipModuleGetFunction(&c->frag_prep[f], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
+    }
+    for (int t = 0; t < kNumFragTiles; ++t) {
+        char name[64];
+        const FragTile& g = kFragTiles[t];
+        snprintf(name, sizeof name, "brik_gemm_frag_%d%d_%dx%d", g.wr, g.wc, g.wa, g.wb);
+        if (hipModuleGetFunction(&c->gemm_frag[t], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
+    }
     if (hipModuleGetFunction(&c->gemmg_adapt[0], c->module, "brik_gemmg_q4_64a") != hipSuccess ||
         hipModuleGetFunction(&c->gemmg_adapt[1], c->module, "brik_gemmg_q4_64aw8") != hipSuccess)
         return bail(BRIK_EMODULE);
@@ -1125,6 +1282,7 @@ void brik_destroy(brik_ctx* c)
     if (c->sws) (void)hipFree(c->sws);
     if (c->cws) (void)hipFree(c->cws);
     if (c->pws) (void)hipFree(c->pws);
+    if (c->fws) (void)hipFree(c->fws);
     if (c->module) (void)hipModuleUnload(c->module);
     delete c;
 }

@@ -2,6 +2,7 @@
 #include "dequant.hip"
 #include "gemv.hip"
 #include "gemm.hip"
+#include "gemm_frag.hip"
 #include "topk.hip"
 #include "quantize.hip"
 #include "conv.hip"

@@ -31,3 +31,6 @@ typedef struct brik_gemv_block {
     uint32_t img_groups;
     uint32_t pad[6];       // 128 bytes
 } brik_gemv_block;
+
+// Rows per staging block of the fragment GEMM (brik_frag_prep_*): 8 up to this K, else 4.
+#define BRIK_FRAG_ROWS8_MAX_K 5120
