@@ -96,6 +96,20 @@ constexpr GemmTile kGemmTiles[] = {{128, 2, 4, 1}, {128, 1, 4, 1}, {128, 3, 4, 1
                                    {64, 1, 4, 3},  {32, 1, 8, 2},  {64, 1, 8, 2}};
 constexpr int kNumGemmTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
+// Few-row GEMM tiles (gemm_few.hip): up to `rows` rows, CW x KW waves, 32 CW columns per block, in the order
+// of BRIK_FEW_TILES.
+// piece_us: time of one piece per k wave; per_cu: blocks a CU holds (registers); both measured.
+struct FewTile {
+    int rows, cw, kw;
+    double piece_us;
+    int per_cu;
+    int bn() const { return 32 * cw; }
+    unsigned threads() const { return 64u * (unsigned)(cw * kw); }
+};
+constexpr FewTile kFewTiles[] = {{8, 1, 4, 2.0, 3}, {16, 1, 4, 2.1, 2}, {16, 2, 4, 2.4, 1}, {32, 4, 1, 1.7, 3}, {64, 4, 1, 2.7, 2}};
+constexpr int kNumFewTiles = sizeof(kFewTiles) / sizeof(kFewTiles[0]);
+constexpr int kFewK = 256;                     // k of one piece (FEW_K)
+
 // Fragment GEMM tiles (gemm_frag.hip): WR x WC waves of WA x WB 32 x 32 blocks each, in the order of
 // BRIK_FRAG_TILES: 192 x 256, 128 x 256, 128 x 128, 64 x 128. `slice_us`: time of a 16-k slice per round of
 // CUs, measured on the product alone. Swept at (M, K, N) = (4096, 9728, 2560), (2048 and 1024, 2560, 9728),
@@ -207,6 +221,7 @@ struct brik_ctx {
     hipFunction_t gemmg_adapt[2] = {};           // brik_gemmg_q4_64a (4 waves), brik_gemmg_q4_64aw8 (8 waves)
     hipFunction_t gemm_f16[kNumGemmTiles] = {};   // f16-weight tiles (TN = 1, PF = 1 only; others null)
     hipFunction_t gemm_sk[3][3] = {};      // split-K few-row kernels, KSL = 2, 4, 8
+    hipFunction_t gemm_few[3][kNumFewTiles] = {};  // brik_gemm_few_<fmt>_<tile>
     hipFunction_t frag_prep[3] = {};             // brik_frag_prep_<fmt>
     hipFunction_t gemm_frag[kNumFragTiles] = {};  // brik_gemm_frag_<tile>
     hipStream_t stream = nullptr;
@@ -489,6 +504,12 @@ unsigned xprep_grid(long rows, long Kp)
 enum SmallMPath { SM_GEMV, SM_SPLITK, SM_TILED };
 constexpr long kSplitKMaxRows = 64;
 
+double tiled_few_us(Fmt f, long M, long K, long N)
+{
+    const double tiled_step = f == F_Q4 ? 0.70 : f == F_Q8 ? 0.83 : 0.86;
+    return 5.0 + std::max(tiled_step * ((K + 255) / 256 * 2), 2.0 * M * N * K / 1e9);
+}
+
 SmallMPath small_m_path(Fmt f, long M, long K, long N)
 {
     const double nk = (double)N * K;
@@ -496,10 +517,9 @@ SmallMPath small_m_path(Fmt f, long M, long K, long N)
                                                                             : nk * (0.375 + 4.0 / kGroup);
     const double steps = (double)((K + 2 * 128 - 1) / (2 * 128) * 2);
     const double gemv_bw = f == F_Q4 ? 7.8e6 : 6.0e6;                   // bytes per us
-    const double tiled_step = f == F_Q4 ? 0.70 : f == F_Q8 ? 0.83 : 0.86;
     const double sk_bw = f == F_Q4 ? 3.4e6 : f == F_Q8 ? 4.8e6 : 2.4e6;
     const double gemv_us = 3.5 + (double)M * (0.35 * std::min(1.0, N / 1024.0) + wbytes / gemv_bw);
-    const double tiled_us = 5.0 + std::max(tiled_step * steps, 2.0 * M * nk / 1e9);
+    const double tiled_us = tiled_few_us(f, M, K, N);
     const double sk_us = M <= kSplitKMaxRows ? 7.7 + 0.15 * steps + wbytes / sk_bw + 0.15 * M : 1e30;
     if (gemv_us <= sk_us && gemv_us <= tiled_us) return SM_GEMV;
     return sk_us <= tiled_us ? SM_SPLITK : SM_TILED;
@@ -588,6 +608,87 @@ int gemm_splitk(brik_ctx* c, Fmt f, const uint16_t* xh, const float* rscale, con
     // the slices' partial tiles, summed in slice order
     size_t n = (size_t)rows * N;
     int ks = (int)p.gz;
+    const size_t blocks = ((n + 3) / 4 + 255) / 256;
+    void* rargs[] = {&part, &y, &n, &ks};
+    return launch(c, K_SPLITK_REDUCE, (unsigned)(blocks < 2048 ? blocks : 2048), 1, 256, 0, rargs);
+}
+
+// Few-row GEMM (gemm_few.hip): dense calls of at most 64 rows, x staged in the launch itself. Tile by rows;
+// K slices over blocks by the modelled time: 4.2 us of launch and ends, `piece_us` per piece of a k wave (x 1.1
+// q8, 1.2 q3; a quarter more per further block on the CU), and with more than one slice 2.7 us for the
+// launch that sums them plus the partial tiles written and read at 2.5 TB/s. Within 10 % at the median of 128
+// measured calls (M 3-64, K 256-9728, N 318-15467).
+struct FewShape {
+    int tile;
+    unsigned gx, ks;
+    int qps;
+    double us;               // modelled time
+};
+
+FewShape few_shape(Fmt f, long rows, int K, int N)
+{
+    FewShape s{};
+    const int pieces = (K + kFewK - 1) / kFewK;
+    s.tile = rows <= 8 ? 0 : rows <= 16 ? (pieces <= 4 ? 1 : 2) : rows <= 32 ? 3 : 4;
+    const FewTile& g = kFewTiles[s.tile];
+    s.gx = (unsigned)((N + g.bn() - 1) / g.bn());
+    const double u = g.piece_us * (f == F_Q4 ? 1.0 : f == F_Q8 ? 1.1 : 1.2);
+    for (int it = (pieces + g.kw - 1) / g.kw; it >= 1; --it) {        // pieces per k wave of a block
+        const int qps = it * g.kw, ks = (pieces + qps - 1) / qps;
+        const int n = (int)(((long)s.gx * ks + kCUs - 1) / kCUs);     // blocks on the fullest CU
+        const int shared = std::min(n, g.per_cu), rounds = (n + g.per_cu - 1) / g.per_cu;
+        double us = 4.2 + rounds * it * u * (1 + 0.25 * (shared - 1));
+        if (ks > 1) us += 2.7 + 8.0 * ks * rows * N / 2.5e6;
+        if (s.ks == 0 || us < s.us) {
+            s.us = us;
+            s.ks = (unsigned)ks;
+            s.qps = qps;
+        }
+    }
+    return s;
+}
+
+size_t few_part_bytes(Fmt f, long rows, int K, int N)
+{
+    const FewShape s = few_shape(f, rows, K, N);
+    return s.ks > 1 ? (size_t)s.ks * rows * N * 4 : 0;
+}
+
+// Whether a dense call takes the few-row GEMM: where its modelled time beats the tiled GEMM's (small_m_path;
+// 10 % and -1.4 us correct what that model gets wrong at short K). It replaces the split-K kernel for every
+// call that would take it: us per call, before -> after: q4 K = 2560, N = 4096, M = 16 14.3 -> 9.3; K = 9728,
+// N = 2560, M = 16 27.4 -> 12.6, M = 64 34.2 -> 21.4; q8 M = 33 35.4 -> 19.2; K = 896, N = 4864, M = 16 9.8 ->
+// 6.1. The tiled GEMM keeps wide matrices past 32 rows (K = 2560, N = 9728, M = 64: 18.5 against 21.6).
+bool use_few(const brik_ctx* c, Fmt f, long rows, int K, int N)
+{
+    if (rows > kSplitKMaxRows || c->opt_tile > 0 || c->opt_splitk == 1) return false;
+    // rows and partial tiles have to fit the no-allocation scratch whoever calls (both entry points take
+    // the same path), and x one buffer resource
+    if (splitk_part_off(rows, K) + few_part_bytes(f, rows, K, N) > BRIK_NOALLOC_SCRATCH_BYTES ||
+        (size_t)rows * K >= (1ull << 29))
+        return false;
+    if (c->opt_splitk == 2) return true;
+    return few_shape(f, rows, K, N).us < 0.9 * tiled_few_us(f, rows, K, N) + 1.4;
+}
+
+int gemm_few(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, const void* sc, const void* mn,
+             float* y, int rows, int K, int N, const Scratch* fixed)
+{
+    const FewShape s = few_shape(f, rows, K, N);
+    float* part = nullptr;
+    if (s.ks > 1) {
+        void* pw = nullptr;
+        if (fixed) pw = static_cast<char*>(fixed->p) + splitk_part_off(rows, K);
+        else HIP_TRY_RC(take_scratch(c, nullptr, c->pws, c->pws_bytes, few_part_bytes(f, rows, K, N), pw));
+        part = static_cast<float*>(pw);
+    }
+    c->last_path = BRIK_PATH_SPLITK;
+    int qps = s.qps;
+    void* args[] = {&x, &p0, &p1, &sc, &mn, &y, &part, &rows, &K, &N, &qps};
+    HIP_TRY_RC(launch_fn(c, c->gemm_few[fmt_index(f)][s.tile], s.gx, s.ks, kFewTiles[s.tile].threads(), 0, args));
+    if (s.ks == 1) return BRIK_OK;
+    size_t n = (size_t)rows * N;
+    int ks = (int)s.ks;
     const size_t blocks = ((n + 3) / 4 + 255) / 256;
     void* rargs[] = {&part, &y, &n, &ks};
     return launch(c, K_SPLITK_REDUCE, (unsigned)(blocks < 2048 ? blocks : 2048), 1, 256, 0, rargs);
@@ -781,6 +882,20 @@ int gemm(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, con
         if (need > fixed->bytes)
             return fail(c, BRIK_EINVAL, "no-allocation call: needs %zu bytes of scratch (staged rows and split-K "
                         "partial tiles), the fixed buffer holds %zu", need, fixed->bytes);
+    }
+    if (!row_off && use_few(c, f, rows, K, N)) {
+        // the workspaces (and the scratch) are held to what the kernels it stands in for need, so that what
+        // a call grows, and what is refused while a graph is captured, does not depend on the choice
+        long Kp;
+        uint16_t* xh;
+        float* rscale;
+        HIP_TRY_RC(gemm_stage_ws(c, rows, K, Kp, xh, rscale, fixed));
+        if (!fixed) {
+            const size_t sk = splitk_part_bytes(c, f, rows, K, N, E);
+            if (sk) HIP_TRY_RC(ensure_buf(c, c->pws, c->pws_bytes, sk));
+        }
+        if (fixed || !c->graph_capturing || c->pws_bytes >= few_part_bytes(f, rows, K, N))
+            return gemm_few(c, f, x, p0, p1, sc, mn, y, rows, K, N, fixed);
     }
     if (!row_off && !fixed && !use_splitk(c, f, rows, K, N, E) && use_frag(c, f, rows, K, N)) {
         bool done = false;
@@ -1227,6 +1342,13 @@ int brik_create(int device, brik_ctx** out)
         snprintf(name, sizeof name, "brik_frag_prep_%s", kFmtNames[f]);
         if (hipModuleGetFunction(&c->frag_prep[f], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
     }
+    for (int f = 0; f < 3; ++f)
+        for (int t = 0; t < kNumFewTiles; ++t) {
+            char name[64];
+            const FewTile& g = kFewTiles[t];
+            snprintf(name, sizeof name, "brik_gemm_few_%s_r%d_%dx%d", kFmtNames[f], g.rows, g.cw, g.kw);
+            if (hipModuleGetFunction(&c->gemm_few[f][t], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
+        }
     for (int t = 0; t < kNumFragTiles; ++t) {
         char name[64];
         const FragTile& g = kFragTiles[t];
