@@ -34,7 +34,7 @@ enum Kern {
     K_CONV_Q8, K_CONV_Q4, K_XPREP_IM2COL, K_CONV_OUT, K_CONV_CHANMAX, K_XPREP_IM2COL3,
     K_GEMV_F16W_V8, K_GEMV_F16W_V4, K_GEMM_F16W,
     K_GEMV_STAGE_Q8, K_GEMV_STAGE_Q4, K_GEMV_STAGE_Q3, K_GEMV_STAGE1_Q4, K_GEMV_STAGE1_Q3,
-    K_SPLITK_REDUCE,
+    K_SPLITK_REDUCE, K_FRAG_ROWS_F16,
     K_COUNT
 };
 
@@ -48,7 +48,7 @@ const char* const kKernelNames[K_COUNT] = {
     "brik_conv_chanmax", "brik_xprep_im2col3_f16",
     "brik_gemv_f16w_v8", "brik_gemv_f16w_v4", "brik_gemm_f16w",
     "brik_gemv_stage_q8", "brik_gemv_stage_q4", "brik_gemv_stage_q3", "brik_gemv_stage1_q4", "brik_gemv_stage1_q3",
-    "brik_splitk_reduce",
+    "brik_splitk_reduce", "brik_frag_rows_f16",
 };
 
 // GEMV variants {team, r, u, d}, in the order of BRIK_GEMV_FMT in gemv.hip: TEAM lanes per row team,
@@ -95,6 +95,19 @@ constexpr GemmTile kGemmTiles[] = {{128, 2, 4, 1}, {128, 1, 4, 1}, {128, 3, 4, 1
                                    {32, 1, 8, 1},  {64, 2, 8, 1},  {32, 1, 8, 4},  {64, 1, 8, 3}, {32, 1, 4, 4},
                                    {64, 1, 4, 3},  {32, 1, 8, 2},  {64, 1, 8, 2}};
 constexpr int kNumGemmTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
+
+// f16-weight GEMM tiles (gemm_frag.hip, brik_gemm_h_*), as kFragTiles: 192 x 256, 256 x 128, 128 x 128, 64 x 64.
+// Fastest of 14 tiles at (M, K, N) = (4096, 9728, 2560) 188 us, (512, 2560, 9728) 34.9, (777, 2560, 4096) 24.6 and
+// (256, 2560, 9728) 23.3, (128, 2560, 2560) 11.6.
+struct HalfTile {
+    int wr, wc, wa, wb;
+    double slice_us;
+    int bm() const { return 32 * wr * wa; }
+    int bn() const { return 32 * wc * wb; }
+    unsigned threads() const { return 64u * (unsigned)(wr * wc); }
+};
+constexpr HalfTile kHalfTiles[] = {{2, 4, 3, 2, 0.32}, {4, 2, 2, 2, 0.21}, {4, 2, 1, 2, 0.135}, {2, 2, 1, 1, 0.055}};
+constexpr int kNumHalfTiles = sizeof(kHalfTiles) / sizeof(kHalfTiles[0]);
 
 // Few-row GEMM tiles (gemm_few.hip): up to `rows` rows, CW x KW waves, 32 CW columns per block, in the order
 // of BRIK_FEW_TILES.
@@ -153,7 +166,7 @@ constexpr long kPrestageMinSets = 2;
 constexpr long kPrestageTailBlocks = 512;
 constexpr long kPlanMinBlocks = 1024;          // grouped-plan blocks, at least (while sets > 1)
 
-enum Fmt { F_Q8 = 8, F_Q4 = 4, F_Q3 = 3 };
+enum Fmt { F_Q8 = 8, F_Q4 = 4, F_Q3 = 3, F_F16 = 16 };   // F_F16: the few-row GEMM only
 
 // LDS bytes of a staged activation row (xprep.h), per group plus one zero group: q8 / q3 96 limb
 // bytes, an f32 sum and an int32 exponent; q4 96 bytes of digit planes and 16 bytes of sums and
@@ -221,7 +234,8 @@ struct brik_ctx {
     hipFunction_t gemmg_adapt[2] = {};           // brik_gemmg_q4_64a (4 waves), brik_gemmg_q4_64aw8 (8 waves)
     hipFunction_t gemm_f16[kNumGemmTiles] = {};   // f16-weight tiles (TN = 1, PF = 1 only; others null)
     hipFunction_t gemm_sk[3][3] = {};      // split-K few-row kernels, KSL = 2, 4, 8
-    hipFunction_t gemm_few[3][kNumFewTiles] = {};  // brik_gemm_few_<fmt>_<tile>
+    hipFunction_t gemm_few[4][kNumFewTiles] = {};  // brik_gemm_few_<fmt>_<tile> (q8, q4, q3, f16)
+    hipFunction_t gemm_h[kNumHalfTiles] = {};     // brik_gemm_h_<tile>
     hipFunction_t frag_prep[3] = {};             // brik_frag_prep_<fmt>
     hipFunction_t gemm_frag[kNumFragTiles] = {};  // brik_gemm_frag_<tile>
     hipStream_t stream = nullptr;
@@ -243,6 +257,7 @@ struct brik_ctx {
     size_t cws_bytes = 0;
     void* pws = nullptr;   // split-K partial tiles [slice][row][column] f32 (grow-only)
     size_t pws_bytes = 0;
+    void* qws = nullptr;   // few-row GEMM: partial tiles (fixed size, so graphs may hold its address)
     void* fws = nullptr;   // fragment GEMM: the dequantized f16 weight panels of one column slab (grow-only)
     size_t fws_bytes = 0;
 
@@ -632,7 +647,7 @@ FewShape few_shape(Fmt f, long rows, int K, int N)
     s.tile = rows <= 8 ? 0 : rows <= 16 ? (pieces <= 4 ? 1 : 2) : rows <= 32 ? 3 : 4;
     const FewTile& g = kFewTiles[s.tile];
     s.gx = (unsigned)((N + g.bn() - 1) / g.bn());
-    const double u = g.piece_us * (f == F_Q4 ? 1.0 : f == F_Q8 ? 1.1 : 1.2);
+    const double u = g.piece_us * (f == F_Q4 || f == F_F16 ? 1.0 : f == F_Q8 ? 1.1 : 1.2);
     for (int it = (pieces + g.kw - 1) / g.kw; it >= 1; --it) {        // pieces per k wave of a block
         const int qps = it * g.kw, ks = (pieces + qps - 1) / qps;
         const int n = (int)(((long)s.gx * ks + kCUs - 1) / kCUs);     // blocks on the fullest CU
@@ -659,15 +674,16 @@ size_t few_part_bytes(Fmt f, long rows, int K, int N)
 // call that would take it: us per call, before -> after: q4 K = 2560, N = 4096, M = 16 14.3 -> 9.3; K = 9728,
 // N = 2560, M = 16 27.4 -> 12.6, M = 64 34.2 -> 21.4; q8 M = 33 35.4 -> 19.2; K = 896, N = 4864, M = 16 9.8 ->
 // 6.1. The tiled GEMM keeps wide matrices past 32 rows (K = 2560, N = 9728, M = 64: 18.5 against 21.6).
-bool use_few(const brik_ctx* c, Fmt f, long rows, int K, int N)
+bool use_few(const brik_ctx* c, Fmt f, long rows, int K, int N, bool fixed)
 {
     if (rows > kSplitKMaxRows || c->opt_tile > 0 || c->opt_splitk == 1) return false;
     // rows and partial tiles have to fit the no-allocation scratch whoever calls (both entry points take
     // the same path), and x one buffer resource
-    if (splitk_part_off(rows, K) + few_part_bytes(f, rows, K, N) > BRIK_NOALLOC_SCRATCH_BYTES ||
-        (size_t)rows * K >= (1ull << 29))
+    const size_t part = few_part_bytes(f, rows, K, N);
+    if (splitk_part_off(rows, K) + part > BRIK_NOALLOC_SCRATCH_BYTES || (size_t)rows * K >= (1ull << 29) ||
+        (part && !fixed && !c->qws))
         return false;
-    if (c->opt_splitk == 2) return true;
+    if (f == F_F16 || c->opt_splitk == 2) return true;
     return few_shape(f, rows, K, N).us < 0.9 * tiled_few_us(f, rows, K, N) + 1.4;
 }
 
@@ -677,15 +693,12 @@ int gemm_few(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1,
     const FewShape s = few_shape(f, rows, K, N);
     float* part = nullptr;
     if (s.ks > 1) {
-        void* pw = nullptr;
-        if (fixed) pw = static_cast<char*>(fixed->p) + splitk_part_off(rows, K);
-        else HIP_TRY_RC(take_scratch(c, nullptr, c->pws, c->pws_bytes, few_part_bytes(f, rows, K, N), pw));
-        part = static_cast<float*>(pw);
+        part = static_cast<float*>(fixed ? static_cast<void*>(static_cast<char*>(fixed->p) + splitk_part_off(rows, K)) : c->qws);
     }
-    c->last_path = BRIK_PATH_SPLITK;
+    if (f != F_F16) c->last_path = BRIK_PATH_SPLITK;
     int qps = s.qps;
     void* args[] = {&x, &p0, &p1, &sc, &mn, &y, &part, &rows, &K, &N, &qps};
-    HIP_TRY_RC(launch_fn(c, c->gemm_few[fmt_index(f)][s.tile], s.gx, s.ks, kFewTiles[s.tile].threads(), 0, args));
+    HIP_TRY_RC(launch_fn(c, c->gemm_few[f == F_F16 ? 3 : fmt_index(f)][s.tile], s.gx, s.ks, kFewTiles[s.tile].threads(), 0, args));
     if (s.ks == 1) return BRIK_OK;
     size_t n = (size_t)rows * N;
     int ks = (int)s.ks;
@@ -883,7 +896,7 @@ int gemm(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, con
             return fail(c, BRIK_EINVAL, "no-allocation call: needs %zu bytes of scratch (staged rows and split-K "
                         "partial tiles), the fixed buffer holds %zu", need, fixed->bytes);
     }
-    if (!row_off && use_few(c, f, rows, K, N)) {
+    if (!row_off && use_few(c, f, rows, K, N, fixed != nullptr)) {
         // the workspaces (and the scratch) are held to what the kernels it stands in for need, so that what
         // a call grows, and what is refused while a graph is captured, does not depend on the choice
         long Kp;
@@ -894,8 +907,7 @@ int gemm(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, con
             const size_t sk = splitk_part_bytes(c, f, rows, K, N, E);
             if (sk) HIP_TRY_RC(ensure_buf(c, c->pws, c->pws_bytes, sk));
         }
-        if (fixed || !c->graph_capturing || c->pws_bytes >= few_part_bytes(f, rows, K, N))
-            return gemm_few(c, f, x, p0, p1, sc, mn, y, rows, K, N, fixed);
+        return gemm_few(c, f, x, p0, p1, sc, mn, y, rows, K, N, fixed);
     }
     if (!row_off && !fixed && !use_splitk(c, f, rows, K, N, E) && use_frag(c, f, rows, K, N)) {
         bool done = false;
@@ -1342,11 +1354,17 @@ int brik_create(int device, brik_ctx** out)
         snprintf(name, sizeof name, "brik_frag_prep_%s", kFmtNames[f]);
         if (hipModuleGetFunction(&c->frag_prep[f], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
     }
-    for (int f = 0; f < 3; ++f)
+    for (int t = 0; t < kNumHalfTiles; ++t) {
+        char name[64];
+        const HalfTile& g = kHalfTiles[t];
+        snprintf(name, sizeof name, "brik_gemm_h_%d%d_%dx%d", g.wr, g.wc, g.wa, g.wb);
+        if (hipModuleGetFunction(&c->gemm_h[t], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
+    }
+    for (int f = 0; f < 4; ++f)
         for (int t = 0; t < kNumFewTiles; ++t) {
             char name[64];
             const FewTile& g = kFewTiles[t];
-            snprintf(name, sizeof name, "brik_gemm_few_%s_r%d_%dx%d", kFmtNames[f], g.rows, g.cw, g.kw);
+            snprintf(name, sizeof name, "brik_gemm_few_%s_r%d_%dx%d", f < 3 ? kFmtNames[f] : "f16", g.rows, g.cw, g.kw);
             if (hipModuleGetFunction(&c->gemm_few[f][t], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
         }
     for (int t = 0; t < kNumFragTiles; ++t) {
@@ -1377,6 +1395,11 @@ int brik_create(int device, brik_ctx** out)
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return bail(BRIK_EHIP);
     if (hipEventCreate(&c->ev_begin) != hipSuccess || hipEventCreate(&c->ev_end) != hipSuccess)
         return bail(BRIK_EHIP);
+    // without it the few-row GEMM runs only the calls that need no partial tiles
+    if (hipMalloc(&c->qws, BRIK_NOALLOC_SCRATCH_BYTES) != hipSuccess) {
+        (void)hipGetLastError();
+        c->qws = nullptr;
+    }
     *out = c;
     return BRIK_OK;
 }
@@ -1405,6 +1428,7 @@ void brik_destroy(brik_ctx* c)
     if (c->cws) (void)hipFree(c->cws);
     if (c->pws) (void)hipFree(c->pws);
     if (c->fws) (void)hipFree(c->fws);
+    if (c->qws) (void)hipFree(c->qws);
     if (c->module) (void)hipModuleUnload(c->module);
     delete c;
 }
@@ -1792,6 +1816,36 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
     uint16_t* xh;
     float* rscale;
     HIP_TRY_RC(gemm_stage_ws(c, M, K, Kp, xh, rscale));
+    if (c->opt_tile == 0) {
+        // the f16-weight GEMM over fragments of x (gemm_frag.hip), or the few-row GEMM where it is modelled
+        // faster; the older kernels below serve forced tiles, and a workspace that holds the plain rows but
+        // not whole panels of 32 (it is not grown here: graphs may hold its address)
+        int S = (K + 31) / 32 * 2, ht = 0;
+        const size_t xbytes = (size_t)((M + 31) / 32) * S * 1024;
+        double h_us = 0;
+        for (int t = 0; t < kNumHalfTiles; ++t) {
+            const HalfTile& g = kHalfTiles[t];
+            const double us = g.slice_us * std::ceil((double)gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()) / kCUs);
+            if (t == 0 || us < h_us) {
+                ht = t;
+                h_us = us;
+            }
+        }
+        h_us = 9.0 + h_us * S;
+        if (M <= kSplitKMaxRows && use_few(c, F_F16, M, K, N, false) && few_shape(F_F16, M, K, N).us < h_us) {
+            const void* none = nullptr;
+            return gemm_few(c, F_F16, x, w, none, none, none, y, M, K, N, nullptr);
+        }
+        if (xbytes + 4 * (size_t)M <= c->ws_bytes && xbytes < (1ull << 31)) {
+            float* rs = reinterpret_cast<float*>(static_cast<char*>(c->ws) + xbytes);
+            const int rpb = K <= BRIK_FRAG_ROWS8_MAX_K ? 8 : 4;
+            void* pargs[] = {&x, &xh, &rs, &Mi, &Ki, &S};
+            HIP_TRY_RC(launch_fn(c, c->fn[K_FRAG_ROWS_F16], (unsigned)((M + rpb - 1) / rpb), 1, 1024, 0, pargs));
+            const HalfTile& g = kHalfTiles[ht];
+            void* args[] = {&xh, &rs, &w, &y, &Mi, &Ni, &Ki, &S};
+            return launch_fn(c, c->gemm_h[ht], gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()), 1, g.threads(), 0, args);
+        }
+    }
     int Kpi = (int)Kp;
     {
         void* args[] = {&x, &xh, &rscale, &Mi, &Ki, &Kpi};

@@ -66,6 +66,20 @@ __device__ __forceinline__ half8_t to_h8(f32x4_t a, f32x4_t b, float up)
     return h;
 }
 
+// The same in natural order (NAT), for f16 weights used as they lie in memory.
+template <bool NAT>
+__device__ __forceinline__ half8_t to_h8_order(f32x4_t a, f32x4_t b, float up)
+{
+    if constexpr (!NAT) return to_h8(a, b, up);
+    half8_t h;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = (_Float16)(a[i] * up);
+        h[4 + i] = (_Float16)(b[i] * up);
+    }
+    return h;
+}
+
 }  // namespace
 
 // ---- 1. activation staging ----------------------------------------------------------------------

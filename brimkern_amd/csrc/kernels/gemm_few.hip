@@ -20,6 +20,7 @@
 // over 128 columns. It took the place of a staging launch, a split-K launch (2-byte scale loads, 32 rows at
 // a time) and the sum: q4 8 x 2560 x 9728 16.1 -> 10.8 us, q8 33 x 9728 x 2560 34.8 -> 18.6 us,
 // q4 16 x 9728 x 2560 27.4 -> 12.6 us, q4 16 x 896 x 4864 9.8 -> 6.1 us.
+// f16 weights (FMT_F16, K % 8 == 0) run the same pieces with no scales, both operands in natural k order.
 #include "common.h"
 
 namespace {
@@ -42,11 +43,29 @@ struct FewPlanes {
     uint32_t colg;                   // flat group index of this lane's column, group 0
     uint32_t glast;                  // last flat group at which 8 groups end inside the plane
     int G, h;
+    uint32_t col;                    // f16: byte offset of this lane's column (and k half) in W
+    int K;
 };
 
 template <int FMT>
 __device__ __forceinline__ void few_load(FewW<FMT>& f, const FewPlanes<FMT>& p, int q)
 {
+    if constexpr (FMT == FMT_F16) {
+        // slice s of step t: halves k = 256 q + 128 t + 16 s + 8 h ..; past K an offset past the buffer's end
+        // (zeros, so an infinite weight of the next row cannot meet x's zero padding)
+        const bool whole = FEW_K * (q + 1) <= p.K;   // uniform
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const int k = 128 * t + 16 * s;
+                const uint32_t off = whole || FEW_K * q + k + 8 * p.h < p.K ? p.col + (uint32_t)(FEW_K * q + k) * 2u : 0xFFFFFF00u;
+                const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(p.r0, off, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) f.c[t].w[4 * s + j] = v[j];
+            }
+        return;
+    }
     const uint32_t start = min(p.colg + (uint32_t)(FEW_G * q), p.glast) * 2u;
     f.s = p.h && FMT != FMT_Q8 ? __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(p.rm, start, 0, 0))
                                : __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(p.rs, start, 0, 0));
@@ -146,7 +165,9 @@ __device__ __forceinline__ void few_body(const float* __restrict__ x, const uint
 
     const size_t wel = (size_t)N * K;
     FewPlanes<FMT> pl;
-    if constexpr (FMT == FMT_Q8) {
+    if constexpr (FMT == FMT_F16) {
+        pl.r0 = make_rsrc(p0, (uint32_t)(wel * 2));
+    } else if constexpr (FMT == FMT_Q8) {
         pl.r0 = make_rsrc(p0, (uint32_t)wel);
     } else if constexpr (FMT == FMT_Q4) {
         pl.r0 = make_rsrc(p0, (uint32_t)(wel / 2));
@@ -155,12 +176,14 @@ __device__ __forceinline__ void few_body(const float* __restrict__ x, const uint
         pl.r1 = make_rsrc(p1, (uint32_t)(wel / 8));
     }
     const uint32_t groups = (uint32_t)((size_t)N * G);
-    pl.rs = make_rsrc(sc, groups * 2);
-    if constexpr (FMT != FMT_Q8) pl.rm = make_rsrc(mn, groups * 2);
+    if constexpr (FMT != FMT_F16) pl.rs = make_rsrc(sc, groups * 2);
+    if constexpr (FMT == FMT_Q4 || FMT == FMT_Q3) pl.rm = make_rsrc(mn, groups * 2);
     pl.colg = (uint32_t)min(ncol, N - 1) * (uint32_t)G;
     pl.glast = groups - FEW_G;
     pl.G = G;
     pl.h = h;
+    pl.col = (uint32_t)min(ncol, N - 1) * (uint32_t)K * 2u + 16u * (uint32_t)h;
+    pl.K = K;
 
     unsigned char* const xb0 = smem + kw * NB * XB;
     float* const rs0 = reinterpret_cast<float*>(smem + MAIN) + kw * NB * XR;
@@ -188,7 +211,7 @@ __device__ __forceinline__ void few_body(const float* __restrict__ x, const uint
             float down;
             const float up = xprep_up(half_max(few_absmax8(xa[i], xc[i])), down);
             if ((lane & 31) == 0) rs0[buf * XR + m] = down;
-            *(half8_t*)(xb + m * XROWP) = to_h8(xa[i], xc[i], up);
+            *(half8_t*)(xb + m * XROWP) = to_h8_order<FMT == FMT_F16>(xa[i], xc[i], up);
         }
     };
 
@@ -199,15 +222,17 @@ __device__ __forceinline__ void few_body(const float* __restrict__ x, const uint
         for (int r = 0; r < 16; ++r) tot[b][r] = 0.f;
     int arow[MB];                                    // LDS byte offset of this lane's A row and k half
 #pragma unroll
-    for (int b = 0; b < MB; ++b) arow[b] = min(32 * b + (lane & 31), M - 1) * XROWP + 128 * h;
+    for (int b = 0; b < MB; ++b) arow[b] = min(32 * b + (lane & 31), M - 1) * XROWP + (FMT == FMT_F16 ? 16 : 128) * h;
     const DeqConst dk = DeqConst::make();
 
     // x before W: loads complete in order, so the rows are converted while the weights are on their way
+    // a k wave without a piece left multiplies zeros: its scales are masked below, f16 weights read as zeros
+    auto piece = [&](int q) { return FMT == FMT_F16 ? (q < q1 ? q : nq) : min(q, nq - 1); };
     FewW<FMT> wq[D];
     load_x(q0 + kw < q1 ? q0 + kw : nq);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int d = 0; d < D; ++d) few_load(wq[d], pl, min(q0 + d * KW + kw, nq - 1));
+    for (int d = 0; d < D; ++d) few_load(wq[d], pl, piece(q0 + d * KW + kw));
     __builtin_amdgcn_sched_barrier(0);
     store_x(0);
     for (int it0 = 0; it0 < iters; it0 += D)
@@ -218,28 +243,30 @@ __device__ __forceinline__ void few_body(const float* __restrict__ x, const uint
         FewW<FMT>& w = wq[d];
         const int q = q0 + it * KW + kw, qn = q + KW, buf = NB == 2 ? it & 1 : 0;
         if constexpr (CW > 1) __syncthreads();       // x of this piece staged; the other buffer free
-        // this piece's scales and mins through the wave's own LDS (lane = plane x column -> any group)
-        *(u32x4_t*)(sb + lane * 16) = w.s;
-        wave_lds_fence();
-        const uint32_t first = pl.colg + (uint32_t)(FEW_G * q);
-        const int shift = (int)(first - min(first, pl.glast));
         WCodes<FMT> cur[2];
+        cur[0] = w.c[0];
+        cur[1] = w.c[1];
+        if constexpr (FMT != FMT_F16) {
+            // this piece's scales and mins through the wave's own LDS (lane = plane x column -> any group)
+            *(u32x4_t*)(sb + lane * 16) = w.s;
+            wave_lds_fence();
+            const uint32_t first = pl.colg + (uint32_t)(FEW_G * q);
+            const int shift = (int)(first - min(first, pl.glast));
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            cur[t] = w.c[t];
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int g = 4 * t + 2 * h + e, at = min(g + shift, FEW_G - 1);
-                const bool live = q < q1 && FEW_G * q + g < G;
-                const uint32_t s = *(const uint16_t*)(sb + (lane & 31) * 16 + at * 2);
-                const uint32_t m = FMT == FMT_Q8 ? 0u : *(const uint16_t*)(sb + 512 + (lane & 31) * 16 + at * 2);
-                cur[t].s[e] = live ? s : 0u;
-                cur[t].m[e] = live ? m : 0u;
-            }
+                for (int e = 0; e < 2; ++e) {
+                    const int g = 4 * t + 2 * h + e, at = min(g + shift, FEW_G - 1);
+                    const bool live = q < q1 && FEW_G * q + g < G;
+                    const uint32_t s = *(const uint16_t*)(sb + (lane & 31) * 16 + at * 2);
+                    const uint32_t m = FMT == FMT_Q8 ? 0u : *(const uint16_t*)(sb + 512 + (lane & 31) * 16 + at * 2);
+                    cur[t].s[e] = live ? s : 0u;
+                    cur[t].m[e] = live ? m : 0u;
+                }
         }
         if (it + 1 < iters) load_x(qn < q1 ? qn : nq);
         __builtin_amdgcn_sched_barrier(0);
-        if (it + D < iters) few_load(w, pl, min(q + D * KW, nq - 1));
+        if (it + D < iters) few_load(w, pl, piece(q + D * KW));
         __builtin_amdgcn_sched_barrier(0);
         floatx16_t acc[MB];
 #pragma unroll
@@ -253,14 +280,20 @@ __device__ __forceinline__ void few_body(const float* __restrict__ x, const uint
         auto read_a16 = [&](half8_t (&a)[MB], int i) {
 #pragma unroll
             for (int b = 0; b < MB; ++b)
-                a[b] = *(const half8_t*)(xb + arow[b] + (i >> 3) * (XR * XROWP) + (i & 7) * 16);
+                a[b] = *(const half8_t*)(xb + arow[b] + (i >> 3) * (XR * XROWP) + (i & 7) * (FMT == FMT_F16 ? 32 : 16));
         };
         half8_t a[2][MB];
         read_a16(a[0], 0);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             if (i < 15) read_a16(a[(i + 1) & 1], i + 1);
-            const half8_t bf = b_frag<FMT>(cur[i >> 3], i < 8 ? go0 : go1, i & 7);
+            half8_t bf;
+            if constexpr (FMT == FMT_F16) {
+                const uint32_t* d = cur[i >> 3].w + 4 * (i & 7);
+                bf = __builtin_bit_cast(half8_t, u32x4_t{d[0], d[1], d[2], d[3]});
+            } else {
+                bf = b_frag<FMT>(cur[i >> 3], i < 8 ? go0 : go1, i & 7);
+            }
 #pragma unroll
             for (int b = 0; b < MB; ++b)
                 acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i & 1][b], bf, acc[b], 0, 0, 0);
@@ -335,3 +368,4 @@ __device__ __forceinline__ void few_body(const float* __restrict__ x, const uint
 BRIK_FEW_TILES(BRIK_GEMM_FEW, q4, FMT_Q4)
 BRIK_FEW_TILES(BRIK_GEMM_FEW, q8, FMT_Q8)
 BRIK_FEW_TILES(BRIK_GEMM_FEW, q3, FMT_Q3)
+BRIK_FEW_TILES(BRIK_GEMM_FEW, f16, FMT_F16)

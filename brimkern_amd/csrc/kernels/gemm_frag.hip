@@ -51,18 +51,45 @@ struct FTile {
 
 // Wait until at most N LDS operations of this wave are outstanding (they complete in issue order; the
 // loop issues no scalar loads).
-// The fragment of row block i at OFF past `base` (row blocks are 4096 bytes apart in an x buffer).
-template <int OFF>
-__device__ __forceinline__ half8_t ds_read_b128_at(uint32_t base, int i)
+// The fragment of block i at OFF past `base`, blocks STRIDE bytes apart.
+template <int STRIDE, int OFF = 0>
+__device__ __forceinline__ half8_t ds_read_b128_by(uint32_t base, int i)
 {
     half8_t v;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(base), "i"(OFF + 4096 * i));
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(base), "i"(OFF + STRIDE * i));
     return v;
 }
 template <int N>
 __device__ __forceinline__ void lds_wait_n()
 {
     asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(N));
+}
+
+// The accumulators times the row scales `rs` (of the tile's rows, in LDS) into y. D layout of a 32 x 32
+// tile: lane holds column lane & 31, register r row 8 (r >> 2) + 4 (lane >> 5) + (r & 3).
+template <class T>
+__device__ __forceinline__ void frag_store(const floatx16_t (&acc)[T::WA][T::WB], const float* rs, float* __restrict__ y,
+                                           int M, int N, int ldy, int mt, int nt, int wr, int wc)
+{
+    const int lane = (int)threadIdx.x & 63, h = lane >> 5;
+    const int m0 = mt * T::BM, n0 = nt * T::BN + wc * T::WB * 32 + (lane & 31);
+#pragma unroll
+    for (int i = 0; i < T::WA; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r0 = 32 * (wr * T::WA + i) + 8 * q + 4 * h;
+            const f32x4_t s4 = *reinterpret_cast<const f32x4_t*>(rs + r0);
+#pragma unroll
+            for (int j = 0; j < T::WB; ++j) {
+                const int n = n0 + 32 * j;
+                if (n >= N) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int m = m0 + r0 + e;
+                    if (m < M) y[(size_t)m * ldy + n] = acc[i][j][4 * q + e] * s4[e];
+                }
+            }
+        }
 }
 
 // One block tile. xf, wf: panels of S fragments (S a multiple of 8); RB, CB: panels of x and of W; y row
@@ -74,7 +101,7 @@ __device__ __forceinline__ void frag_tile_run(unsigned char* smem, const uint16_
                                               int mt, int nt)
 {
     constexpr int WA = T::WA, WB = T::WB, XQ = T::XQ, AL = T::AL;
-    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave / T::WC, wc = wave % T::WC;
     const brsrc_t rx = make_rsrc(xf, (uint32_t)((size_t)RB * S * 1024));
@@ -140,7 +167,7 @@ __device__ __forceinline__ void frag_tile_run(unsigned char* smem, const uint16_
     if (tid < T::BM) store_rscale(lds_addr(smem + XQ * T::XBUF) + 4 * (uint32_t)tid, rs_row);
     const uint32_t abase = lds_addr(smem) + (uint32_t)(wr * WA * 4096) + voff;
 #pragma unroll
-    for (int i = 0; i < WA; ++i) a[i] = ds_read_b128_at<0>(abase, i);
+    for (int i = 0; i < WA; ++i) a[i] = ds_read_b128_by<4096>(abase, i);
 
     // Step t multiplies x buffer xq. At slice 2 the wave waits for its own x loads of step t + 1 and meets
     // the others: after that step t + 1 may be read and the buffer of step t - 1 refilled (step
@@ -183,8 +210,8 @@ __device__ __forceinline__ void frag_tile_run(unsigned char* smem, const uint16_
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     }
-                    a[i] = s == 0 ? ds_read_b128_at<1024>(anext, i) : s == 1 ? ds_read_b128_at<2048>(anext, i)
-                         : s == 2 ? ds_read_b128_at<3072>(anext, i) : ds_read_b128_at<0>(anext, i);
+                    a[i] = s == 0 ? ds_read_b128_by<4096, 1024>(anext, i) : s == 1 ? ds_read_b128_by<4096, 2048>(anext, i)
+                         : s == 2 ? ds_read_b128_by<4096, 3072>(anext, i) : ds_read_b128_by<4096>(anext, i);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -198,26 +225,7 @@ __device__ __forceinline__ void frag_tile_run(unsigned char* smem, const uint16_
     for (int i = 0; i < WA; ++i) tie(a[i]);
     wait_vm<0>();
 
-    // D layout of a 32x32 tile: lane holds column lane & 31, register r row 8 (r >> 2) + 4 h + (r & 3)
-    const float* const rs = reinterpret_cast<const float*>(smem + XQ * T::XBUF);
-    const int m0 = mt * T::BM, n0 = nt * T::BN + wc * WB * 32 + (lane & 31);
-#pragma unroll
-    for (int i = 0; i < WA; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int r0 = 32 * (wr * WA + i) + 8 * q + 4 * h;
-            const f32x4_t s4 = *reinterpret_cast<const f32x4_t*>(rs + r0);
-#pragma unroll
-            for (int j = 0; j < WB; ++j) {
-                const int n = n0 + 32 * j;
-                if (n >= N) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int m = m0 + r0 + e;
-                    if (m < M) y[(size_t)m * ldy + n] = acc[i][j][4 * q + e] * s4[e];
-                }
-            }
-        }
+    frag_store<T>(acc, reinterpret_cast<const float*>(smem + XQ * T::XBUF), y, M, N, ldy, mt, nt, wr, wc);
 }
 
 // Tile (row, column) of block b: blocks are dealt to the 8 XCDs round-robin, so each XCD takes a run of
@@ -255,12 +263,15 @@ static_assert(FRAG_CH * 1024 == BRIK_FRAG_ROWS8_MAX_K, "rows per staging block")
 
 // Halves offset of 8-element chunk c (k = 8 c ..) of row r of panel rb: step c >> 4 of 128 k, lane half
 // (c >> 3) & 1, slice c & 7 (gemm.hip's k mapping).
+// NAT: slice c >> 1, half c & 1 (k = 16 s + 8 h + i), the f16-weight mapping.
+template <bool NAT>
 __device__ __forceinline__ size_t frag_chunk_at(int rb, int r, int c, int S)
 {
+    if constexpr (NAT) return ((size_t)rb * S + (c >> 1)) * 512 + (c & 1) * 256 + r * 8;
     return ((size_t)rb * S + 8 * (c >> 4) + (c & 7)) * 512 + ((c >> 3) & 1) * 256 + r * 8;
 }
 
-template <int R>
+template <int R, bool NAT = false>
 __device__ __forceinline__ void frag_rows(const float* __restrict__ x, uint16_t* __restrict__ xf,
                                           float* __restrict__ rscale, int g, int M, int K, int S, float (*wmax)[8])
 {
@@ -297,7 +308,7 @@ __device__ __forceinline__ void frag_rows(const float* __restrict__ x, uint16_t*
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
         const int c = c0 + C * i;
-        if (c < nchp) *(half8_t*)(xf + frag_chunk_at(rb, rr, c, S)) = to_h8(v[i][0], v[i][1], up);
+        if (c < nchp) *(half8_t*)(xf + frag_chunk_at<NAT>(rb, rr, c, S)) = to_h8_order<NAT>(v[i][0], v[i][1], up);
     }
     for (int c = c0 + C * CH; c < nchp; c += C) {
         f32x4_t p = {0.f, 0.f, 0.f, 0.f}, q = p;
@@ -305,7 +316,7 @@ __device__ __forceinline__ void frag_rows(const float* __restrict__ x, uint16_t*
             p = *(const f32x4_t*)(xr + c * 8);
             q = *(const f32x4_t*)(xr + c * 8 + 4);
         }
-        *(half8_t*)(xf + frag_chunk_at(rb, rr, c, S)) = to_h8(p, q, up);
+        *(half8_t*)(xf + frag_chunk_at<NAT>(rb, rr, c, S)) = to_h8_order<NAT>(p, q, up);
     }
 }
 
@@ -373,6 +384,191 @@ __device__ __forceinline__ void frag_prep(const float* __restrict__ x, uint16_t*
     frag_dequant<FMT>(p0, p1, sc, mn, wf, n0, N, K, cb, item % T, S);
 }
 
+
+// ---- f16 weights ----------------------------------------------------------------------------------
+// The same product with W as given, [N, K] f16 rows (the reference's MATMUL_T_F16W, shaders.ts:2240-2259):
+// re-laying W out would read and write it once more, so its rows go through LDS beside x, 32 k (64 bytes) of
+// each row and step, by direct loads of 16 rows each, XQ - 2 steps ahead. The 16-byte chunk c of row r sits
+// at chunk c ^ ((r >> 2) & 3) of its 64 bytes, so the 16 rows of a read phase touch all 64 banks. Both
+// operands are in natural order: slice s, half h, element i is k = 16 s + 8 h + i.
+// The tiled GEMM's f16 form loaded each W row 16 bytes per lane straight into registers, so a load touched 32
+// lines, and its steps waited for them: 0.6 us and more per 128 k whatever the rows. What bounds this one
+// is LDS (192 x 256 tile, per slice of 384 MFMA clocks: 40 KiB read, 14 KiB written) and, for small tiles,
+// the load latency, hence 32-k steps and as many in flight as fit: 64-k steps in three buffers ran
+// 256 x 128 at 42 us where six 32-k buffers run 34.9 (512 x 2560 x 9728). Per call, before -> after:
+// M = 512, K = 2560, N = 9728 56 -> 40 us; M = 4096, K = 9728, N = 2560 421 -> 246 us (product 188 us,
+// 1.08 PFLOP/s); M = 128, K = 2560, N = 1024 48 -> 16 us. Few rows (gemm_few.hip): M = 8, K = 9728, N = 2560
+// 150 -> 15.6 us.
+template <int WR_, int WC_, int WA_, int WB_, int XQ_>
+struct HTile {
+    static constexpr int WR = WR_, WC = WC_, WA = WA_, WB = WB_, XQ = XQ_;
+    static constexpr int NW = WR * WC, NT = 64 * NW;
+    static constexpr int BMB = WR * WA, BNB = WC * WB;
+    static constexpr int BM = 32 * BMB, BN = 32 * BNB;
+    static constexpr int XBUF = BMB * 2048, BUF = (BMB + BNB) * 2048;      // bytes of a step: x, then W rows
+    // direct loads per wave and step (1 KiB pieces dealt round-robin; a wave without a last piece repeats it)
+    static constexpr int AL = (BMB * 2 + NW - 1) / NW, BL = (BNB * 2 + NW - 1) / NW, LD = AL + BL;
+    static constexpr int SMEM = XQ * BUF + BM * 4;
+    static_assert(XQ >= 3 && SMEM <= 160 * 1024 && WA - 1 + WB <= 15 && (XQ - 2) * LD < 64, "tile");
+};
+
+template <class T>
+__device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t* __restrict__ xf,
+                                             const float* __restrict__ rscale, const uint16_t* __restrict__ w,
+                                             float* __restrict__ y, int M, int N, int K, int S, int RB, int mt, int nt)
+{
+    constexpr int WA = T::WA, WB = T::WB, XQ = T::XQ, LD = T::LD;
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave / T::WC, wc = wave % T::WC;
+    const brsrc_t rx = make_rsrc(xf, (uint32_t)((size_t)RB * S * 1024));
+    const brsrc_t rw = make_rsrc(w, (uint32_t)((size_t)N * K * 2));
+    const uint32_t voff = (uint32_t)lane * 16;
+    const int steps = S / 2, full = K / 32;          // full: steps of 32 live k
+
+    uint32_t xbase[T::AL], woff[T::BL], xdst[T::AL], wdst[T::BL];
+#pragma unroll
+    for (int i = 0; i < T::AL; ++i) {
+        const int q = min(T::NW * i + wave, T::BMB * 2 - 1);
+        xbase[i] = (uint32_t)(min(mt * T::BMB + (q >> 1), RB - 1) * S + (q & 1)) * 1024u;
+        xdst[i] = (uint32_t)q * 1024u;
+    }
+#pragma unroll
+    for (int i = 0; i < T::BL; ++i) {
+        const int q = min(T::NW * i + wave, T::BNB * 2 - 1), r = 16 * q + (lane >> 2);
+        woff[i] = (uint32_t)min(nt * T::BN + r, N - 1) * (uint32_t)K * 2u + (uint32_t)(((lane & 3) ^ ((r >> 2) & 3)) * 16);
+        wdst[i] = (uint32_t)(T::XBUF + q * 1024);
+    }
+    auto load = [&](int u, int step, uint32_t buf) {
+        if (u < T::AL)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void_t*)(smem + buf + xdst[u]), 16, voff,
+                                                     (int)(xbase[u] + (uint32_t)step * 2048u), 0, 0);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void_t*)(smem + buf + wdst[u - T::AL]), 16,
+                                                     woff[u - T::AL], step * 64, 0, 0);
+    };
+
+    const float rs_row = tid < T::BM ? rscale[min(mt * T::BM + tid, M - 1)] : 0.f;
+    half8_t a[WA], b[2][WB];
+    floatx16_t acc[WA][WB];
+#pragma unroll
+    for (int i = 0; i < WA; ++i)
+#pragma unroll
+        for (int j = 0; j < WB; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+#pragma unroll
+    for (int q = 0; q < XQ - 1; ++q)
+#pragma unroll
+        for (int u = 0; u < LD; ++u) load(u, min(q, steps - 1), (uint32_t)(q * T::BUF));
+    wait_vm<(XQ - 2) * LD>();                        // step 0
+    step_barrier();
+    if (tid < T::BM) store_rscale(lds_addr(smem + XQ * T::BUF) + 4 * (uint32_t)tid, rs_row);
+    const uint32_t abase = lds_addr(smem) + (uint32_t)(wr * WA * 2048) + voff;
+    uint32_t boff[2];                                // W fragment of slice s: row lane & 31, chunk 2 s + h
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+        boff[s] = lds_addr(smem) + T::XBUF + (uint32_t)(wc * WB * 2048 + (lane & 31) * 64) +
+                  (uint32_t)(((2 * s + h) ^ ((lane >> 2) & 3)) * 16);
+#pragma unroll
+    for (int j = 0; j < WB; ++j) b[0][j] = ds_read_b128_by<2048>(boff[0], j);
+#pragma unroll
+    for (int i = 0; i < WA; ++i) a[i] = ds_read_b128_by<2048>(abase, i);
+    // every LDS and scalar operation so far: the loop's counted waits then count LDS reads alone
+    lds_wait();
+
+    // Step t multiplies buffer xq; at slice 1 the wave waits for its loads of step t + 1 and meets the others,
+    // then loads step t + XQ - 1 into the buffer of step t - 1. W fragments are read a slice ahead, x
+    // fragments into the registers of the row just multiplied.
+    uint32_t xq = 0;
+    for (int t = 0; t < full; ++t) {
+        const uint32_t x1 = xq + 1 == (uint32_t)XQ ? 0u : xq + 1, xfill = xq == 0 ? (uint32_t)XQ - 1 : xq - 1;
+        const int fill = min(t + XQ - 1, steps - 1);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int cur = s, nxt = s ^ 1;
+            const uint32_t nb = (s == 1 ? x1 : xq) * T::BUF;
+            if (s == 1) {
+                wait_vm<(XQ - 3) * LD>();
+                asm volatile("s_barrier" ::: "memory");
+            }
+#pragma unroll
+            for (int i = 0; i < WA; ++i) {
+                if (i == 0) {
+                    lds_wait_n<WA - 1>();
+#pragma unroll
+                    for (int j = 0; j < WB; ++j) tie(b[cur][j]);
+                } else {
+                    lds_wait_n<WA - 1 + WB>();
+                }
+                tie(a[i]);
+                if (i == 0) {
+#pragma unroll
+                    for (int j = 0; j < WB; ++j) b[nxt][j] = ds_read_b128_by<2048>(boff[nxt] + nb, j);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < WB; ++j) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[cur][j], acc[i][j], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (s == 1) {
+                        const int o = i * WB + j;
+#pragma unroll
+                        for (int u = o * LD / (WA * WB); u < (o + 1) * LD / (WA * WB); ++u) load(u, fill, xfill * T::BUF);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                a[i] = s == 0 ? ds_read_b128_by<2048, 1024>(abase + nb, i) : ds_read_b128_by<2048>(abase + nb, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        xq = x1;
+    }
+    lds_wait();
+#pragma unroll
+    for (int i = 0; i < WA; ++i) tie(a[i]);
+#pragma unroll
+    for (int j = 0; j < WB; ++j) tie(b[0][j]);
+    wait_vm<0>();
+    if (steps > full) {
+        // the last step's K - 32 full live k: chunks past K hold another row's values, taken as zeros
+        lds_barrier();                               // every wave's loads of the step have landed
+        const uint32_t nb = xq * T::BUF;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (32 * full + 16 * s >= K) break;
+            const bool live = 32 * full + 16 * s + 8 * h < K;
+            half8_t bt[WB];
+#pragma unroll
+            for (int j = 0; j < WB; ++j) {
+                u32x4_t v = *(const u32x4_t*)(smem + nb + (boff[s] - lds_addr(smem)) + 2048 * j);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = live ? v[e] : 0u;
+                bt[j] = __builtin_bit_cast(half8_t, v);
+            }
+#pragma unroll
+            for (int i = 0; i < WA; ++i) {
+                const half8_t at = *(const half8_t*)(smem + nb + wr * WA * 2048 + lane * 16 + 1024 * s + 2048 * i);
+#pragma unroll
+                for (int j = 0; j < WB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(at, bt[j], acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+    frag_store<T>(acc, reinterpret_cast<const float*>(smem + XQ * T::BUF), y, M, N, N, mt, nt, wr, wc);
+}
+
+template <class T>
+__device__ __forceinline__ void f16_gemm(const uint16_t* __restrict__ xf, const float* __restrict__ rscale,
+                                         const uint16_t* __restrict__ w, float* __restrict__ y, int M, int N, int K,
+                                         int S)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[T::SMEM];
+    int mt, nt;
+    frag_tile_of((int)blockIdx.x, (M + T::BM - 1) / T::BM, (N + T::BN - 1) / T::BN, mt, nt);
+    f16_tile_run<T>(smem, xf, rscale, w, y, M, N, K, S, (M + 31) / 32, mt, nt);
+}
+
 }  // namespace
 
 #define BRIK_FRAG_PREP(FMTN, FMT)                                                                         \
@@ -399,3 +595,27 @@ BRIK_FRAG_PREP(q4, FMT_Q4) BRIK_FRAG_PREP(q8, FMT_Q8) BRIK_FRAG_PREP(q3, FMT_Q3)
 #define BRIK_FRAG_TILES(X) X(2, 4, 3, 2, 4, 4) X(1, 8, 4, 1, 4, 8) X(1, 4, 4, 1, 4, 8) X(1, 4, 2, 1, 4, 8)
 #endif
 BRIK_FRAG_TILES(BRIK_GEMM_FRAG)
+
+// Rows of x in natural order for the f16-weight GEMM (S slices of 16 k per panel, zeros past K).
+extern "C" __global__ __launch_bounds__(1024, 8) void brik_frag_rows_f16(const float* __restrict__ x,
+                                                                         uint16_t* __restrict__ xf,
+                                                                         float* __restrict__ rscale, int M, int K,
+                                                                         int S)
+{
+    __shared__ float wmax[16][8];
+    if (K <= BRIK_FRAG_ROWS8_MAX_K) frag_rows<8, true>(x, xf, rscale, (int)blockIdx.x, M, K, S, wmax);
+    else frag_rows<4, true>(x, xf, rscale, (int)blockIdx.x, M, K, S, wmax);
+}
+
+// f16-weight GEMM kernels: brik_gemm_h_<WR><WC>_<WA>x<WB>, in the order of the runtime's table (kHalfTiles).
+#define BRIK_GEMM_H(WR, WC, WA, WB, XQ)                                                                   \
+    extern "C" __global__ __launch_bounds__(64 * WR * WC) void brik_gemm_h_##WR##WC##_##WA##x##WB(        \
+        const uint16_t* __restrict__ xf, const float* __restrict__ rscale, const uint16_t* __restrict__ w, \
+        float* __restrict__ y, int M, int N, int K, int S)                                                \
+    {                                                                                                     \
+        f16_gemm<HTile<WR, WC, WA, WB, XQ>>(xf, rscale, w, y, M, N, K, S);                                \
+    }
+#ifndef BRIK_HALF_TILES
+#define BRIK_HALF_TILES(X) X(2, 4, 3, 2, 5) X(4, 2, 2, 2, 6) X(4, 2, 1, 2, 5) X(2, 2, 1, 1, 9)
+#endif
+BRIK_HALF_TILES(BRIK_GEMM_H)

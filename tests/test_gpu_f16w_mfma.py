@@ -1,0 +1,71 @@
+"""The f16-weight product on the matrix cores: the few-row GEMM (2 to 64 rows) and the GEMM over x fragments
+with W rows through LDS (gemm_frag.hip), each tile of both, against the oracle at the matmul bar (1e-3 of
+sum |x w|). K ends at every remainder of 32 that the entry point takes there (multiples of 8), so the last
+step's chunks past K, which hold the next row's values, have to count as zeros: an infinite weight at the
+start of a row must not reach the row before it.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from helpers import Gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def gpu(ctx):
+    g = Gpu(ctx)
+    yield g
+    g.free()
+
+
+def data(M, K, N, seed):
+    rng = np.random.default_rng(seed)
+    x = (rng.standard_normal((M, K)) * np.exp2(np.arange(M) % 37 - 18)[:, None]).astype(np.float32)
+    return x, (rng.standard_normal((N, K)) * 0.05).astype(np.float16)
+
+
+def run(gpu, x, w):
+    (M, K), N = x.shape, w.shape[0]
+    yb = gpu.up(np.full(M * N, np.nan, np.float32))
+    gpu.ctx.matmul_t_f16w(gpu.up(x), gpu.up(w.view(np.uint16)), yb, M, K, N)
+    return gpu.ctx.download(yb, np.float32, M * N).reshape(M, N)
+
+
+def check(y, x, w):
+    ref, den = O.matmul_t_f16w(x.ravel(), w.view(np.uint16).ravel(), *x.shape, w.shape[0])
+    assert np.all(np.abs(y - ref) <= 1e-3 * den + 1e-30)
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (4096, 288, 2560), (4095, 72, 2555),      # 192 x 256
+    (512, 520, 9728), (500, 64, 9701),        # 256 x 128
+    (777, 1000, 4096), (770, 32, 4090),       # 128 x 128
+    (130, 40, 333), (65, 8, 70), (200, 1048, 129), (100, 10248, 65),   # 64 x 64; one chunk of K; rows read twice
+])
+def test_h_tiles(gpu, M, K, N):
+    x, w = data(M, K, N, M + K)
+    y = run(gpu, x, w)
+    check(y, x, w)
+    assert np.array_equal(y.view(np.uint32), run(gpu, x, w).view(np.uint32))
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 8, 33), (8, 1032, 127), (9, 264, 129), (16, 2568, 200), (17, 40, 130),
+                                   (32, 1304, 257), (24, 5152, 65), (33, 24, 513), (64, 544, 127), (47, 3104, 130)])
+def test_few_f16(gpu, M, K, N):
+    x, w = data(M, K, N, M + K + 1)
+    check(run(gpu, x, w), x, w)
+
+
+@pytest.mark.parametrize("M", [5, 40, 200])
+@pytest.mark.parametrize("K", [40, 64, 72, 88])
+def test_infinite_weight_stays_in_its_row(gpu, M, K):
+    N = 70
+    x, w = data(M, K, N, 7)
+    x = np.abs(x) + np.float32(0.5)
+    w[7, 0] = w[69, K - 1] = np.float16(np.inf)
+    y = run(gpu, x, w)
+    cols = [n for n in range(N) if n not in (7, 69)]
+    assert np.isposinf(y[:, [7, 69]]).all() and np.isfinite(y[:, cols]).all()
+    check(y[:, cols], x, np.ascontiguousarray(w[cols]))
