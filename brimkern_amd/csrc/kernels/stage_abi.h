@@ -34,3 +34,7 @@ typedef struct brik_gemv_block {
 
 // Rows per staging block of the fragment GEMM (brik_frag_prep_*): 8 up to this K, else 4.
 #define BRIK_FRAG_ROWS8_MAX_K 5120
+
+// Most taps (kh kw) of the tap-by-tap convolution GEMM (conv_gemm.hip): its weight staging holds 2 KiB per
+// tap in LDS, its product a row of scales per tap.
+#define BRIK_CONV_GEMM_MAX_TAPS 25
