@@ -1740,7 +1740,8 @@ bool conv_gemm_plan(brik_ctx* c, long Cin, long HW, long Cout, long taps, long P
         for (long ks = 1; ks <= 16 && ks <= T; ++ks) {
             const long sps = (T + ks - 1) / ks;
             if ((T + sps - 1) / sps != ks) continue;
-            if (ks > 1 && (size_t)ks * Cout * P * 4 > BRIK_NOALLOC_SCRATCH_BYTES) break;
+            // the partial tiles lie in the context's fixed buffer, which a create short of memory goes without
+            if (ks > 1 && (!c->qws || (size_t)ks * Cout * P * 4 > BRIK_NOALLOC_SCRATCH_BYTES)) break;
             // blocks of 64 x 64 share a CU two at a time, so their time grows with their number; slices cost
             // the sum's launch and the partial tiles
             const double per = (double)tiles * ks / kCUs, load = t == 0 ? std::max(1.0, 1.06 * per) : std::ceil(per);
