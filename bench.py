@@ -431,7 +431,7 @@ def conv_f4(ctx, steps, warmup):
         ctx.free(bb)
     out["shape"] = "Cin 320, 64x64, Cout 320, 3x3, stride 1, pad 1, q4 weight"
     out["frac_of_mfma_peak"] = round(out["implicit_gemm"]["TFLOPs"] / MFMA_F16_PEAK_TFLOPS, 4)
-    out["launches"] = "brik_conv_chanmax + brik_xprep_im2col3_f16 + brik_gemm_q4 (stores [Cout, pixels] + bias)"
+    out["launches"] = "brik_conv_prep_q4 + brik_gemm_conv_42_1x2 + brik_splitk_reduce"
     return out
 
 
@@ -457,7 +457,7 @@ def f16w_f4(ctx, steps, warmup, cache_bytes=768 << 20):
                         "frac": round(b1 / (ms1 * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "copies": copies},
             "gemm_M512": {"us": round(msm * 1e3, 2), "TFLOPs": round(tf, 1),
                           "frac": round(tf / MFMA_F16_PEAK_TFLOPS, 4)},
-            "kernels": "brik_gemv_f16w_v8 (M = 1); brik_xprep_f16 + brik_gemm_f16_96x1w8 (M = 512)"}
+            "kernels": "brik_gemv_f16w_v8 (M = 1); brik_frag_rows_f16 + brik_gemm_h_42_2x2 (M = 512)"}
 
 
 def gemm_cfg4(ctx, steps, warmup):
