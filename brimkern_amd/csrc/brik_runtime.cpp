@@ -1060,8 +1060,8 @@ int matmul(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, c
 // ---- sampling pre-work -------------------------------------------------------------------------
 
 constexpr int kTopkMax = 64;                      // BRIK_TOPK_MAX, TOPK_MAX in topk.hip
-size_t topk_blocks(int n) { return ((size_t)n + 4095) / 4096; }          // 4 waves x 1024 logits
-size_t topk_maxima(int n) { return 256 * topk_blocks(n); }                // one per lane (16 logits)
+size_t topk_blocks(int n) { return ((size_t)n + 1023) / 1024; }          // prep blocks (4 logits per thread)
+size_t topk_maxima(int n) { return 64 * topk_blocks(n); }                 // one per 16 logits
 // workspace: lane maxima, then the LM-head logits
 size_t topk_logits_off(int n) { return (4 * topk_maxima(n) + 255) / 256 * 256; }
 

@@ -7,9 +7,9 @@
 // The reference's top_k runs in one 128-thread workgroup and is exact unless more than 8 of the true
 // top-k share an id mod 128. Here the selection is exact for every input, and ties are ordered by
 // id (smaller first), on a (value, id) key that is unique per element. Two launches:
-//   a. brik_topk_prep: each block takes 4096 logits, applies the softcap and the penalty (the recent
-//      ids of its range are marked in an LDS bitmap), writes them back, and every lane writes the
-//      maximum of its 16 consecutive logits ("lane maxima": maximum q covers logits [16q, 16q + 16)).
+//   a. brik_topk_prep: each block takes 1024 logits, applies the softcap and the penalty (the recent
+//      ids of its range are marked in an LDS bitmap), writes them back, and every four lanes write the
+//      maximum of their 16 consecutive logits ("lane maxima": maximum q covers logits [16q, 16q + 16)).
 //      A q4 / q3 LM head staged once per call runs these passes in its own epilogue instead
 //      (gemv.hip, brik_gemvh_*), with the same maxima layout.
 //   b. brik_topk_select, one block: folds the lane maxima into 256 maxima of disjoint element sets and
@@ -27,7 +27,7 @@ namespace {
 
 constexpr int TOPK_MAX = 64;
 constexpr int TOPK_CAP = 8192;      // candidate list capacity (keys)
-constexpr int TOPK_BLOCK = 4096;    // logits per block: 4 waves x 64 lanes x 16
+constexpr int TOPK_BLOCK = 1024;    // logits per block: 4 waves x 64 lanes x 4
 
 // The order key of common.h (NaN -> 0).
 __device__ __forceinline__ uint32_t okey(float v) { return order_key(v); }
@@ -63,8 +63,10 @@ __device__ __forceinline__ void bitonic_desc(K* s, int P)
 
 }  // namespace
 
-// Block b: logits [4096 b, 4096 b + 4096); thread t: the 16 consecutive logits 4096 b + 16 t + j and
-// lane maximum q = 256 b + t.
+// Block b: logits [1024 b, 1024 b + 1024); thread t: the 4 consecutive logits 1024 b + 4 t + j; four threads
+// share lane maximum q = 64 b + t / 4. Bound by latency: one load, then the softcap's tanhf of each value in
+// turn. With 16 logits per thread the launch was 38 blocks for 151936 logits, every lane's 16 bytes in a cache
+// line of their own; now 149 blocks of contiguous loads, 6.96 -> 4.77 us (head and passes 51.7 -> 48.2 us).
 extern "C" __global__ __launch_bounds__(256) void brik_topk_prep(float* __restrict__ logits, int n, float cap,
                                                                  const int32_t* __restrict__ recent, int n_recent,
                                                                  float penalty, int pen,
@@ -73,8 +75,24 @@ extern "C" __global__ __launch_bounds__(256) void brik_topk_prep(float* __restri
     __shared__ uint32_t marks[TOPK_BLOCK / 32];
     const int tid = threadIdx.x;
     const long base = (long)blockIdx.x * TOPK_BLOCK;
+    // the logits first, in flight beside the marks: one 16-byte buffer load of a whole chunk (the logits
+    // need only 4-byte alignment), else one at a time
+    float raw[4];
+    const long c0 = base + 4 * tid;
+    if (c0 + 4 <= n) {
+        const brsrc_t r = make_rsrc(logits, (uint32_t)n * 4u);
+        const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, (uint32_t)c0 * 4u, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t w = v[e];          // a scalar first: bit_cast of v[e] itself read element 0
+            raw[e] = __builtin_bit_cast(float, w);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) raw[j] = c0 + j < n ? logits[c0 + j] : 0.f;
+    }
     if (pen) {
-        for (int i = tid; i < TOPK_BLOCK / 32; i += 256) marks[i] = 0u;
+        if (tid < TOPK_BLOCK / 32) marks[tid] = 0u;
         __syncthreads();
         // ids outside [0, n) are skipped, as sampleNextToken does (src/lib/webgpu/sampling.ts:86)
         for (int r = tid; r < n_recent; r += 256) {
@@ -86,29 +104,10 @@ extern "C" __global__ __launch_bounds__(256) void brik_topk_prep(float* __restri
         }
         __syncthreads();
     }
-    // all 16 loads of a thread first (one memory round trip; four at a time took four): four 16-byte
-    // buffer loads of a whole chunk (the logits need only 4-byte alignment), else one at a time
-    float raw[16];
-    const long c0 = base + 16 * tid;
-    if (c0 + 16 <= n) {
-        const brsrc_t r = make_rsrc(logits, (uint32_t)n * 4u);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, (uint32_t)(c0 + 4 * u) * 4u, 0, 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t w = v[e];      // a scalar first: bit_cast of v[e] itself read element 0
-                raw[4 * u + e] = __builtin_bit_cast(float, w);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) raw[j] = c0 + j < n ? logits[c0 + j] : 0.f;
-    }
     uint32_t m = 0u;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int o = 16 * tid + j;
+    for (int j = 0; j < 4; ++j) {
+        const int o = 4 * tid + j;
         const long i = base + o;
         if (i < n) {
             float v = raw[j];
@@ -119,13 +118,15 @@ extern "C" __global__ __launch_bounds__(256) void brik_topk_prep(float* __restri
             m = max(m, okey(v));
         }
     }
-    maxima[(long)blockIdx.x * 256 + tid] = m;
+    m = max(m, (uint32_t)__shfl_xor((int)m, 1));
+    m = max(m, (uint32_t)__shfl_xor((int)m, 2));
+    if ((tid & 3) == 0) maxima[(long)blockIdx.x * 64 + (tid >> 2)] = m;
 }
 
 constexpr int TOPK_LANES = 2048;    // lanes read back by the select block, at most
 constexpr int TOPK_STAGE = 16384;   // lane maxima staged in LDS (vectors of up to 262144 logits)
 
-// One block of 1024 threads; m = the number of lane maxima (256 per prep block, or one per 16 logits
+// One block of 1024 threads; m = the number of lane maxima (64 per prep block, or one per 16 logits
 // from a fused LM head), maximum q covering logits [16 q, 16 q + 16).
 extern "C" __global__ __launch_bounds__(1024) void brik_topk_select(const float* __restrict__ logits, int n, int k,
                                                                     const uint32_t* __restrict__ maxima, int m,
