@@ -241,7 +241,7 @@ extern "C" __global__ __launch_bounds__(1024) void brik_conv_chanmax(const float
 
 // The pixel's row scale from the channel maxima of its in-image taps (as brik_xprep_f16 scales a row).
 __device__ __forceinline__ float im2col_scale(const float* __restrict__ cmax, int y0, int x0, int H, int W, int kh,
-                                              int kw, int& e)
+                                              int kw, float& down)
 {
     // every load in range (clamped coordinates) and unconditional, a tap outside the image then
     // dropped: the loads issue together instead of one guarded round trip each
@@ -254,9 +254,7 @@ __device__ __forceinline__ float im2col_scale(const float* __restrict__ cmax, in
             mx = fmaxf(mx, (iy >= 0 && iy < H && ix >= 0 && ix < W) ? c : 0.f);
         }
     }
-    e = 15;                                                        // zero / non-finite rows: scale 1
-    if (mx > 0.f && mx <= 3.4028235e38f) (void)frexpf(mx, &e);    // mx = f * 2^e, f in [0.5, 1)
-    return ldexpf(1.f, 15 - e);
+    return xprep_up(mx, down);
 }
 
 constexpr int IM2COL_CPT = 8;    // chunks of 8 elements per thread
@@ -273,9 +271,9 @@ extern "C" __global__ __launch_bounds__(256) void brik_xprep_im2col_f16(
     const int m = min((int)blockIdx.x * 64 + lane, M - 1);
     const int oy = m / OW, ox = m % OW, kk = kh * kw;
     const int y0 = oy * stride - pad, x0 = ox * stride - pad;
-    int e;
-    const float up = im2col_scale(cmax, y0, x0, H, W, kh, kw, e);
-    if (blockIdx.y == 0 && w == 0 && (int)blockIdx.x * 64 + lane < M) rscale[m] = ldexpf(1.f, e - 15);
+    float down;
+    const float up = im2col_scale(cmax, y0, x0, H, W, kh, kw, down);
+    if (blockIdx.y == 0 && w == 0 && (int)blockIdx.x * 64 + lane < M) rscale[m] = down;
     const int nchp = Kp / 8;
     const int c0 = (blockIdx.y * 4 + w) * IM2COL_CPT;              // the same for the whole wave
     // Taps through a buffer resource: the per-thread offset is the pixel's corner (y0, x0), the tap's
@@ -354,9 +352,9 @@ extern "C" __global__ __launch_bounds__(64 * IM2COL3_WAVES) void brik_xprep_im2c
     const int m = min((int)blockIdx.x * 64 + lane, M - 1);        // rows past M: row M - 1, not written
     const int oy = m / OW, ox = m % OW;
     const int y0 = oy * stride - pad, x0 = ox * stride - pad;
-    int e;
-    const float up = im2col_scale(cmax, y0, x0, H, W, 3, 3, e);
-    if (blockIdx.y == 0 && w == 0 && (int)blockIdx.x * 64 + lane < M) rscale[m] = ldexpf(1.f, e - 15);
+    float down;
+    const float up = im2col_scale(cmax, y0, x0, H, W, 3, 3, down);
+    if (blockIdx.y == 0 && w == 0 && (int)blockIdx.x * 64 + lane < M) rscale[m] = down;
     // taps through a buffer resource starting pad rows and columns before the input (see the generic
     // form); the host keeps every offset below 2^31
     const int lead = pad * W + pad;
