@@ -139,9 +139,9 @@ __device__ __forceinline__ void few_load(FewW<FMT>& f, const FewPlanes<FMT>& p, 
 #pragma unroll
     for (int t = 0; t < C::PARTS; ++t) {
         const uint32_t at = p.off + (uint32_t)((C::PARTS * q + t) * C::PB);
-        // f16: chunks past K get an offset past the buffer's end (zeros, so an infinite weight of the next row
+        // f16: chunks past K get an offset past the buffer's end (N K < 2^31 halves; zeros, so an infinite weight of the next row
         // cannot meet x's zero padding); the other formats' dead groups have their scales masked
-        const uint32_t dead = FMT == FMT_F16 && FEW_K * q + 128 * t + 8 * ((int)(threadIdx.x & 63) % C::LPR) >= p.K ? 0xFFFFFF00u : 0u;
+        const uint32_t dead = FMT == FMT_F16 && FEW_K * q + 128 * t + 8 * ((int)(threadIdx.x & 63) % C::LPR) >= p.K ? 0xFFFFFFF0u : 0u;
 #pragma unroll
         for (int i = 0; i < C::NI; ++i)
             f.c[t][i] = __builtin_amdgcn_raw_buffer_load_b128(p.r0, (at + (uint32_t)i * p.step) | dead, 0, 0);

@@ -439,6 +439,16 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
         woff[i] = (uint32_t)min(nt * T::BN + r, N - 1) * (uint32_t)K * 2u + (uint32_t)(((lane & 3) ^ ((r >> 2) & 3)) * 16);
         wdst[i] = (uint32_t)(T::XBUF + q * 1024);
     }
+    // Before the loads of the last step when it is not whole: its chunks past K get an offset past the end of W
+    // (N K < 2^31 halves), as a vector offset, because the range check of a buffer load leaves the scalar one
+    // out; they would otherwise run up to 48 bytes past the last row.
+    auto cut_last = [&]() {
+#pragma unroll
+        for (int i = 0; i < T::BL; ++i) {
+            const int r = 16 * min(T::NW * i + wave, T::BNB * 2 - 1) + (lane >> 2);
+            if (32 * full + 8 * ((lane & 3) ^ ((r >> 2) & 3)) >= K) woff[i] = 0xFFFFFFF0u;
+        }
+    };
     auto load = [&](int u, int step, uint32_t buf) {
         if (u < T::AL)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void_t*)(smem + buf + xdst[u]), 16, voff,
@@ -458,9 +468,12 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 #pragma unroll
-    for (int q = 0; q < XQ - 1; ++q)
+    for (int q = 0; q < XQ - 1; ++q) {
+        const int step = min(q, steps - 1);
+        if (step == full) cut_last();                // uniform
 #pragma unroll
-        for (int u = 0; u < LD; ++u) load(u, min(q, steps - 1), (uint32_t)(q * T::BUF));
+        for (int u = 0; u < LD; ++u) load(u, step, (uint32_t)(q * T::BUF));
+    }
     wait_vm<(XQ - 2) * LD>();                        // step 0
     step_barrier();
     if (tid < T::BM) store_rscale(lds_addr(smem + XQ * T::BUF) + 4 * (uint32_t)tid, rs_row);
@@ -484,6 +497,7 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
     for (int t = 0; t < full; ++t) {
         const uint32_t x1 = xq + 1 == (uint32_t)XQ ? 0u : xq + 1, xfill = xq == 0 ? (uint32_t)XQ - 1 : xq - 1;
         const int fill = min(t + XQ - 1, steps - 1);
+        if (fill == full) cut_last();                // uniform; the whole steps are all loaded by then
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int cur = s, nxt = s ^ 1;
@@ -531,7 +545,7 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
     for (int j = 0; j < WB; ++j) tie(b[0][j]);
     wait_vm<0>();
     if (steps > full) {
-        // the last step's K - 32 full live k: chunks past K hold another row's values, taken as zeros
+        // the last step's K - 32 full live k: chunks past K were not loaded and are taken as zeros
         lds_barrier();                               // every wave's loads of the step have landed
         const uint32_t nb = xq * T::BUF;
 #pragma unroll

@@ -69,3 +69,12 @@ def test_infinite_weight_stays_in_its_row(gpu, M, K):
     cols = [n for n in range(N) if n not in (7, 69)]
     assert np.isposinf(y[:, [7, 69]]).all() and np.isfinite(y[:, cols]).all()
     check(y[:, cols], x, np.ascontiguousarray(w[cols]))
+
+
+@pytest.mark.parametrize("M,K", [(40, 40), (100, 40), (100, 72), (300, 88), (2000, 72)])
+def test_weights_that_end_their_allocation(gpu, M, K):
+    """W of whole 64 KiB in an allocation of its own: the last row's last step has 8, 16 or 24 of 32 k inside."""
+    N = 4096
+    assert N * K * 2 % 65536 == 0
+    x, w = data(M, K, N, M * K)
+    check(run(gpu, x, w), x, w)
