@@ -493,61 +493,50 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
     // Step t multiplies buffer xq; at slice 1 the wave waits for its loads of step t + 1 and meets the others,
     // then loads step t + XQ - 1 into the buffer of step t - 1. W fragments are read a slice ahead, x
     // fragments into the registers of the row just multiplied.
-    // The loop stops once where the next load is that of the cut step.
     uint32_t xq = 0;
-    int t = 0, stop = steps > full ? max(full - (XQ - 1), 0) : full;
-    while (true) {
-        for (; t < stop; ++t) {
-            const uint32_t x1 = xq + 1 == (uint32_t)XQ ? 0u : xq + 1, xfill = xq == 0 ? (uint32_t)XQ - 1 : xq - 1;
-            const int fill = min(t + XQ - 1, steps - 1);
+    for (int t = 0; t < full; ++t) {
+        const uint32_t x1 = xq + 1 == (uint32_t)XQ ? 0u : xq + 1, xfill = xq == 0 ? (uint32_t)XQ - 1 : xq - 1;
+        const int fill = min(t + XQ - 1, steps - 1);
+        if (fill == full) cut_last();                // uniform; the whole steps are all loaded by then
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int cur = s, nxt = s ^ 1;
-                const uint32_t nb = (s == 1 ? x1 : xq) * T::BUF;
-                if (s == 1) {
-                    wait_vm<(XQ - 3) * LD>();
-                    asm volatile("s_barrier" ::: "memory");
-                }
-#pragma unroll
-                for (int i = 0; i < WA; ++i) {
-                    if (i == 0) {
-                        lds_wait_n<WA - 1>();
-#pragma unroll
-                        for (int j = 0; j < WB; ++j) tie(b[cur][j]);
-                    } else {
-                        lds_wait_n<WA - 1 + WB>();
-                    }
-                    tie(a[i]);
-                    if (i == 0) {
-#pragma unroll
-                        for (int j = 0; j < WB; ++j) b[nxt][j] = ds_read_b128_by<2048>(boff[nxt] + nb, j);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int j = 0; j < WB; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[cur][j], acc[i][j], 0, 0, 0);
-                        __builtin_amdgcn_sched_barrier(0);
-                        if (s == 1) {
-                            const int o = i * WB + j;
-#pragma unroll
-                            for (int u = o * LD / (WA * WB); u < (o + 1) * LD / (WA * WB); ++u) load(u, fill, xfill * T::BUF);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-                    a[i] = s == 0 ? ds_read_b128_by<2048, 1024>(abase + nb, i) : ds_read_b128_by<2048>(abase + nb, i);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+        for (int s = 0; s < 2; ++s) {
+            const int cur = s, nxt = s ^ 1;
+            const uint32_t nb = (s == 1 ? x1 : xq) * T::BUF;
+            if (s == 1) {
+                wait_vm<(XQ - 3) * LD>();
+                asm volatile("s_barrier" ::: "memory");
             }
-            xq = x1;
+#pragma unroll
+            for (int i = 0; i < WA; ++i) {
+                if (i == 0) {
+                    lds_wait_n<WA - 1>();
+#pragma unroll
+                    for (int j = 0; j < WB; ++j) tie(b[cur][j]);
+                } else {
+                    lds_wait_n<WA - 1 + WB>();
+                }
+                tie(a[i]);
+                if (i == 0) {
+#pragma unroll
+                    for (int j = 0; j < WB; ++j) b[nxt][j] = ds_read_b128_by<2048>(boff[nxt] + nb, j);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < WB; ++j) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[cur][j], acc[i][j], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (s == 1) {
+                        const int o = i * WB + j;
+#pragma unroll
+                        for (int u = o * LD / (WA * WB); u < (o + 1) * LD / (WA * WB); ++u) load(u, fill, xfill * T::BUF);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                a[i] = s == 0 ? ds_read_b128_by<2048, 1024>(abase + nb, i) : ds_read_b128_by<2048>(abase + nb, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        if (stop == full) break;                     // uniform
-        lds_wait();                                  // the fragments in flight first: moves may not touch them before
-#pragma unroll
-        for (int i = 0; i < WA; ++i) tie(a[i]);
-#pragma unroll
-        for (int j = 0; j < WB; ++j) tie(b[0][j]);
-        cut_last();
-        stop = full;
+        xq = x1;
     }
     lds_wait();
 #pragma unroll
