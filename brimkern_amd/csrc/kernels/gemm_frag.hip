@@ -439,23 +439,18 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
         woff[i] = (uint32_t)min(nt * T::BN + r, N - 1) * (uint32_t)K * 2u + (uint32_t)(((lane & 3) ^ ((r >> 2) & 3)) * 16);
         wdst[i] = (uint32_t)(T::XBUF + q * 1024);
     }
-    // Before the loads of the last step when it is not whole: its chunks past K get an offset past the end of W
-    // (N K < 2^31 halves), as a vector offset, because the range check of a buffer load leaves the scalar one
-    // out; they would otherwise run up to 48 bytes past the last row.
-    auto cut_last = [&]() {
-#pragma unroll
-        for (int i = 0; i < T::BL; ++i) {
-            const int r = 16 * min(T::NW * i + wave, T::BNB * 2 - 1) + (lane >> 2);
-            if (32 * full + 8 * ((lane & 3) ^ ((r >> 2) & 3)) >= K) woff[i] = 0xFFFFFFF0u;
-        }
-    };
+    // W's step is in its vector offset, moved on by each load: the range check of a buffer load leaves the scalar
+    // offset out, and the last step of the last row may run up to 48 bytes past the end of W. Steps past the last
+    // read a next row's values or nothing.
     auto load = [&](int u, int step, uint32_t buf) {
         if (u < T::AL)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void_t*)(smem + buf + xdst[u]), 16, voff,
                                                      (int)(xbase[u] + (uint32_t)step * 2048u), 0, 0);
-        else
+        else {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void_t*)(smem + buf + wdst[u - T::AL]), 16,
-                                                     woff[u - T::AL], step * 64, 0, 0);
+                                                     woff[u - T::AL], 0, 0, 0);
+            woff[u - T::AL] += 64;
+        }
     };
 
     const float rs_row = tid < T::BM ? rscale[min(mt * T::BM + tid, M - 1)] : 0.f;
@@ -468,12 +463,9 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 #pragma unroll
-    for (int q = 0; q < XQ - 1; ++q) {
-        const int step = min(q, steps - 1);
-        if (step == full) cut_last();                // uniform
+    for (int q = 0; q < XQ - 1; ++q)
 #pragma unroll
-        for (int u = 0; u < LD; ++u) load(u, step, (uint32_t)(q * T::BUF));
-    }
+        for (int u = 0; u < LD; ++u) load(u, min(q, steps - 1), (uint32_t)(q * T::BUF));
     wait_vm<(XQ - 2) * LD>();                        // step 0
     step_barrier();
     if (tid < T::BM) store_rscale(lds_addr(smem + XQ * T::BUF) + 4 * (uint32_t)tid, rs_row);
@@ -497,7 +489,6 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
     for (int t = 0; t < full; ++t) {
         const uint32_t x1 = xq + 1 == (uint32_t)XQ ? 0u : xq + 1, xfill = xq == 0 ? (uint32_t)XQ - 1 : xq - 1;
         const int fill = min(t + XQ - 1, steps - 1);
-        if (fill == full) cut_last();                // uniform; the whole steps are all loaded by then
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int cur = s, nxt = s ^ 1;
@@ -545,7 +536,7 @@ __device__ __forceinline__ void f16_tile_run(unsigned char* smem, const uint16_t
     for (int j = 0; j < WB; ++j) tie(b[0][j]);
     wait_vm<0>();
     if (steps > full) {
-        // the last step's K - 32 full live k: chunks past K were not loaded and are taken as zeros
+        // the last step's K - 32 full live k: chunks past K hold a next row's values or none, taken as zeros
         lds_barrier();                               // every wave's loads of the step have landed
         const uint32_t nb = xq * T::BUF;
 #pragma unroll
