@@ -30,6 +30,7 @@ SIGNATURES = {
     "brik_destroy": (None, [_P]),
     "brik_last_error": (ctypes.c_char_p, [_P]),
     "brik_last_path": (_I, [_P]),
+    "brik_last_kernel": (ctypes.c_char_p, [_P]),
     "brik_strerror": (ctypes.c_char_p, [_I]),
     "brik_device_count": (_I, [ctypes.POINTER(_I)]),
     "brik_alloc": (_I, [_P, _Z, ctypes.POINTER(_P)]),
@@ -258,6 +259,10 @@ class Context:
     def last_path(self) -> int:
         """BRIK_PATH_* of the last matmul call on this context (0 before any, or for K = 0)."""
         return self.lib.brik_last_path(self.handle)
+
+    def last_kernel(self) -> str:
+        """The product kernel of the last matmul or convolution, by the stem of its name (brik_last_kernel)."""
+        return self.lib.brik_last_kernel(self.handle).decode()
 
     def timer_begin(self):
         self._check(self.lib.brik_timer_begin(self.handle))

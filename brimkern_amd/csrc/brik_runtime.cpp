@@ -285,6 +285,7 @@ struct brik_ctx {
     size_t scratch_bytes = 0;
     int scratch_err = 0;
     int last_path = 0;            // BRIK_PATH_* of the last matmul call (brik_last_path)
+    const char* last_kernel = ""; // product kernel of the last matmul or convolution (brik_last_kernel)
     bool graph_capturing = false;
     bool graph_used_ws = false;   // the open capture recorded a launch on a context workspace
     // bumped whenever a context workspace is freed and reallocated (ensure_buf): a graph recorded
@@ -703,6 +704,7 @@ int gemm_few(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1,
         part = static_cast<float*>(fixed ? static_cast<void*>(static_cast<char*>(fixed->p) + splitk_part_off(rows, K)) : c->qws);
     }
     if (f != F_F16) c->last_path = BRIK_PATH_SPLITK;
+    c->last_kernel = "gemm_few";
     int qps = s.qps;
     void* args[] = {&x, &p0, &p1, &sc, &mn, &y, &part, &rows, &K, &N, &qps};
     HIP_TRY_RC(launch_fn(c, c->gemm_few[f == F_F16 ? 3 : fmt_index(f)][s.tile], s.gx, s.ks, kFewTiles[s.tile].threads(), 0, args));
@@ -733,12 +735,14 @@ int gemm_run(brik_ctx* c, Fmt f, const uint16_t* xh, const float* rscale, const 
 {
     if (use_splitk(c, f, rows, K, N, E)) {
         c->last_path = BRIK_PATH_SPLITK;
+        c->last_kernel = "gemm_sk";
         HIP_TRY_RC(gemm_splitk(c, f, xh, rscale, p0, p1, sc, mn, y, rows, K, N, row_off, E, fixed));
         if (!pair) return BRIK_OK;
         return gemm_splitk(c, f, xh, rscale, pair->p0, p1, pair->sc, pair->mn, pair->y, rows, K, N, row_off, E,
                            fixed);
     }
     c->last_path = BRIK_PATH_TILED;
+    c->last_kernel = row_off ? "gemmg" : "gemm";
     int Mi = rows, Ki = K, Ni = N, Ei = E;
     const int t = gemm_tile(c, rows, N, K, E);
     const GemmTile& gt = kGemmTiles[t];
@@ -868,6 +872,7 @@ int gemm_frag(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1
     if (!ensure_fws(c, s.wbytes)) return BRIK_OK;
     done = true;
     c->last_path = BRIK_PATH_TILED;
+    c->last_kernel = "gemm_frag";
     uint16_t* xf = static_cast<uint16_t*>(c->ws);
     float* rscale = reinterpret_cast<float*>(static_cast<char*>(c->ws) + (size_t)s.RB * s.S * 1024);
     uint16_t* wf = static_cast<uint16_t*>(c->fws);
@@ -1002,6 +1007,7 @@ int matmul(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, c
            HeadArgs* head = nullptr)
 {
     c->last_path = 0;
+    c->last_kernel = "";
     if (K == 0) return fill_zero(c, y, (size_t)M * N);   // empty sums, whatever the path
     // A large q4 / q3 matrix at M = 1 (an LM head) stages x once per call (brik_gemv_stage1_<fmt>, one
     // block) and its blocks copy the image instead of each staging x themselves. q8 measured no gain.
@@ -1039,6 +1045,7 @@ int matmul(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, c
             HIP_TRY_RC(launch(c, f == F_Q4 ? K_GEMV_STAGE1_Q4 : K_GEMV_STAGE1_Q3, 1, 1, kStageThreads, 0, sargs));
         }
         c->last_path = stage1 ? BRIK_PATH_GEMV_STAGED : BRIK_PATH_GEMV;
+        c->last_kernel = "gemv";
         if (head && stage1 && v == kHeadVariant) {
             // the LM head with the top-k pre-work in its epilogue: its LDS adds the row sums of a block
             // and a bitmap of its rows
@@ -1295,6 +1302,8 @@ const char* brik_strerror(int code)
 const char* brik_last_error(const brik_ctx* c) { return c ? c->err : "null context"; }
 
 int brik_last_path(const brik_ctx* c) { return c ? c->last_path : 0; }
+
+const char* brik_last_kernel(const brik_ctx* c) { return c ? c->last_kernel : ""; }
 
 int brik_device_count(int* count)
 {
@@ -1600,6 +1609,7 @@ static int moe(brik_ctx* c, const char* who, const float* x, const int32_t* row_
 {
     if (!c) return BRIK_EINVAL;
     c->last_path = 0;
+    c->last_kernel = "";
     if (E < 0 || R < 0) return fail(c, BRIK_EINVAL, "%s: negative E=%d or R=%d", who, E, R);
     int r = check_mm(c, who, x, nib, nullptr, sc, mn, y, R, K, N, F_Q4);
     if (r == BRIK_OK && pair)
@@ -1765,6 +1775,7 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
                   int stride, int pad)
 {
     if (!c) return BRIK_EINVAL;
+    c->last_kernel = "";
     if (Cin < 1 || H < 1 || W < 1 || Cout < 1 || kh < 1 || kw < 1 || stride < 1 || pad < 0)
         return fail(c, BRIK_EINVAL, "%s: bad shape Cin=%d H=%d W=%d Cout=%d kernel %dx%d stride %d pad %d", who, Cin,
                     H, W, Cout, kh, kw, stride, pad);
@@ -1792,6 +1803,7 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
     if (!use_gemm) {
         // 256 output pixels x 16 output channels per block (conv.hip, conv_direct)
         const unsigned gx = (unsigned)((M + 255) / 256), gy = (unsigned)((Cout + 15) / 16);
+        c->last_kernel = "conv2d_direct";
         if (f == F_Q8) {
             void* args[] = {&inp, &p0, &sc, &bias, &out, &Ci, &Hi, &Wi, &Co, &khi, &kwi, &si, &pi, &OHi, &OWi};
             return launch(c, K_CONV_Q8, gx, gy, 256, 0, args);
@@ -1823,6 +1835,7 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
         if (room || ensure_fws(c, cg.wbytes)) {
             if (!room) wf = static_cast<uint16_t*>(c->fws);
             c->last_path = BRIK_PATH_TILED;
+            c->last_kernel = "gemm_conv";
             int taps = kh * kw, xblocks = (HW + 15) / 16, P = rows;
             void* pargs[] = {&inp, &xt, &xs, &p0, &sc, &mn, &wf, &Ci, &HW, &Co, &taps, &xblocks};
             HIP_TRY_RC(launch_fn(c, c->conv_prep[f == F_Q4],
@@ -1880,6 +1893,7 @@ int brik_conv2d_q4(brik_ctx* c, const float* inp, const uint8_t* nib, const uint
 int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y, int M, int K, int N)
 {
     if (!c) return BRIK_EINVAL;
+    c->last_kernel = "";
     if (M < 0 || K < 0 || N < 0) return fail(c, BRIK_EINVAL, "matmul_t_f16w: negative shape M=%d K=%d N=%d", M, K, N);
     if (K % 4) return fail(c, BRIK_EINVAL, "matmul_t_f16w: K=%d is not a multiple of 4", K);
     if (M == 0 || N == 0) return BRIK_OK;
@@ -1901,6 +1915,7 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
     if (use_gemv) {
         const long sets = ((long)N + 7) / 8;
         const unsigned gx = (unsigned)(sets < 16384 ? sets : 16384);
+        c->last_kernel = "gemv_f16w";
         void* args[] = {&x, &w, &y, &Ki, &Ni};
         return launch(c, K % 8 ? K_GEMV_F16W_V4 : K_GEMV_F16W_V8, gx, (unsigned)M, 256, (size_t)K * 4, args);
     }
@@ -1934,6 +1949,7 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
             void* pargs[] = {&x, &xh, &rs, &Mi, &Ki, &S};
             HIP_TRY_RC(launch_fn(c, c->fn[K_FRAG_ROWS_F16], (unsigned)((M + rpb - 1) / rpb), 1, 1024, 0, pargs));
             const HalfTile& g = kHalfTiles[ht];
+            c->last_kernel = "gemm_h";
             void* args[] = {&xh, &rs, &w, &y, &Mi, &Ni, &Ki, &S};
             return launch_fn(c, c->gemm_h[ht], gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()), 1, g.threads(), 0, args);
         }
@@ -1965,6 +1981,7 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
             }
         }
         const GemmTile& g = kGemmTiles[best];
+        c->last_kernel = "gemm_f16";
         const void* none = nullptr;
         const int* no_rows = nullptr;
         int Ei = 0, trans = 0;
@@ -1974,6 +1991,7 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
                          targs);
     }
     // K % 32 != 0: the LDS-tiled kernel (K steps of 32 with zero-filled tails)
+    c->last_kernel = "gemm_f16w";
     void* args[] = {&xh, &rscale, &w, &y, &Mi, &Ki, &Ni, &Kpi};
     return launch(c, K_GEMM_F16W, (unsigned)((N + 127) / 128), (unsigned)((M + 63) / 64), 256, 0, args);
 }

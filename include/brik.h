@@ -384,6 +384,12 @@ int brik_set_option(brik_ctx *ctx, int key, int value);
 #define BRIK_PATH_SPLITK 4       /* few-row split-K MFMA GEMM (partial tiles summed in slice order) */
 int brik_last_path(const brik_ctx *ctx);
 
+/* The product kernel behind it, by the stem of its name without brik_ ("" before any call, or for K = 0):
+ * gemv, gemm (tiled), gemmg (expert-grouped), gemm_sk (split-K), gemm_few (few rows), gemm_frag (fragments);
+ * gemv_f16w, gemm_h, gemm_f16, gemm_f16w for f16 weights (and gemm_few); gemm_conv (tap by tap), gemm or
+ * gemm_sk (im2col rows), conv2d_direct for convolutions. A diagnostic as brik_last_path. */
+const char *brik_last_kernel(const brik_ctx *ctx);
+
 #ifdef __cplusplus
 }
 #endif

@@ -29,7 +29,7 @@ def gpu(ctx):
 
 def run(gpu, fmt, t, x, M):
     y = gpu.matmul(fmt, x, gpu.planes(fmt, t), M, t["K"], t["N"])
-    assert gpu.ctx.last_path() == BRIK_PATH_SPLITK
+    assert gpu.ctx.last_path() == BRIK_PATH_SPLITK and gpu.ctx.last_kernel() == "gemm_few"
     r, den = getattr(O, f"matmul_t_{fmt}")(x, *[t[k] for k in PLANES[fmt]], M, t["K"], t["N"], absden=True)
     return y, r, den
 
