@@ -265,7 +265,7 @@ struct brik_ctx {
     void* pws = nullptr;   // split-K partial tiles [slice][row][column] f32 (grow-only)
     size_t pws_bytes = 0;
     void* qws = nullptr;   // few-row GEMM: partial tiles (fixed size, so graphs may hold its address)
-    void* fws = nullptr;   // fragment GEMM: the dequantized f16 weight panels of one column slab (grow-only)
+    void* fws = nullptr;   // fragment GEMM: x panels and the f16 weight panels of one column slab (grow-only)
     size_t fws_bytes = 0;
 
     // pinned staging ring of brik_h2d_async (allocated on first use): uploads in flight as
@@ -483,21 +483,19 @@ size_t gemm_stage_bytes(long rows, long K, long& Kp)
     return (size_t)rows * Kp * 2 + 4 * (size_t)rows;
 }
 
-// Bytes of `rows` rows as fragment panels (32 rows, K padded to 128) and their row scales.
-size_t frag_stage_bytes(long rows, long K) { return (size_t)((rows + 31) / 32) * ((K + 127) / 128 * 8) * 1024 + 4 * (size_t)rows; }
-
-// Workspace for `rows` staged f16 activation rows of K (padded to Kp) and their row scales.
+// Workspace for `rows` staged f16 activation rows of K (padded to Kp) and their row scales. `want`: the size it
+// takes if it has to grow (and that much can be had).
 int gemm_stage_ws(brik_ctx* c, int rows, int K, long& Kp, uint16_t*& xh, float*& rscale,
-                  const Scratch* fixed = nullptr)
+                  const Scratch* fixed = nullptr, size_t want = 0)
 {
     const size_t bytes = gemm_stage_bytes(rows, K, Kp);
     const size_t xbytes = (size_t)rows * Kp * 2;
     if (xbytes >= (1ull << 31))
         return fail(c, BRIK_EINVAL, "matmul: %d rows x K=%d exceed the 2 GiB staged-activation limit", rows, K);
     void* p = nullptr;
-    // when the workspace has to grow, by enough for the fragment GEMM's whole panels of 32 rows too
-    const size_t want = !fixed && c->ws_bytes < bytes ? std::max(bytes, frag_stage_bytes(rows, K)) : bytes;
-    HIP_TRY_RC(take_scratch(c, fixed, c->ws, c->ws_bytes, want, p));
+    if (!fixed && c->ws_bytes < bytes && want > bytes && ensure_buf(c, c->ws, c->ws_bytes, want) != BRIK_OK)
+        (void)hipGetLastError();               // what is needed will do
+    HIP_TRY_RC(take_scratch(c, fixed, c->ws, c->ws_bytes, bytes, p));
     xh = static_cast<uint16_t*>(p);
     rscale = reinterpret_cast<float*>(static_cast<char*>(p) + xbytes);
     return BRIK_OK;
@@ -773,7 +771,7 @@ int gemm_run(brik_ctx* c, Fmt f, const uint16_t* xh, const float* rscale, const 
     return launch_fn(c, fn, blocks, 1, gt.threads(), 0, args);
 }
 
-// The weight slab `fws`, grown to at least `bytes`. No graph holds it (its users check), so unlike the other
+// The fragment workspace `fws`, grown to at least `bytes`. No graph holds it (its users check), so unlike the other
 // workspaces its growth leaves recorded graphs valid.
 bool ensure_fws(brik_ctx* c, size_t bytes)
 {
@@ -798,7 +796,7 @@ bool ensure_fws(brik_ctx* c, size_t bytes)
 struct FragShape {
     long S, RB, CB;             // fragments per panel (K padded to 128), panels of x and of W
     long slab;                  // W panels per column slab
-    size_t xbytes, wbytes;      // workspaces: x fragments and row scales, one slab of W fragments
+    size_t xbytes, wbytes;      // x fragments and row scales (whole 256 bytes), one slab of W fragments
 };
 
 FragShape frag_shape(long M, long K, long N)
@@ -808,7 +806,7 @@ FragShape frag_shape(long M, long K, long N)
     s.RB = (M + 31) / 32;
     s.CB = (N + 31) / 32;
     s.slab = std::max(8L, (long)(kFragSlabBytes / ((size_t)s.S * 1024)) / 8 * 8);
-    s.xbytes = frag_stage_bytes(M, K);
+    s.xbytes = ((size_t)s.RB * s.S * 1024 + 4 * (size_t)M + 255) & ~(size_t)255;
     s.wbytes = (size_t)std::min(s.slab, s.CB) * s.S * 1024;
     return s;
 }
@@ -839,13 +837,10 @@ int frag_tile(long M, long N)
 // staging costs more than it saves (q4 K = 2560, N = 9728, M = 512: 41 against 47).
 bool use_frag(brik_ctx* c, Fmt f, long M, long K, long N)
 {
-    // a captured call keeps the tiled GEMM (the same bits), so that no graph holds the W panels' address;
-    // and the row staging must fit where the tiled GEMM's would have, so that no workspace grows that
-    // would not have grown
+    // a captured call keeps the tiled GEMM (the same bits), so that no graph holds the W panels' address
     if (c->opt_tile > 0 || c->graph_capturing || K > 65536) return false;
     const FragShape s = frag_shape(M, K, N);
-    long Kp;
-    if (s.xbytes >= (1ull << 31) || (c->ws_bytes < s.xbytes && c->ws_bytes >= gemm_stage_bytes(M, K, Kp))) return false;
+    if (s.xbytes >= (1ull << 31)) return false;               // x panels: one buffer resource
     constexpr double kSliceUs[kNumFragTiles] = {0.28, 0.178, 0.086, 0.056};   // per round, as fitted
     const double mk = (double)M * K, nk = (double)N * K, mn = (double)M * N;
     const double wb = f == F_Q4 ? 0.625 : f == F_Q8 ? 1.0625 : 0.5;
@@ -862,20 +857,25 @@ bool use_frag(brik_ctx* c, Fmt f, long M, long K, long N)
     return frag_us < 0.93 * tiled_us;
 }
 
-// Returns BRIK_OK with `done` false when the workspaces could not be had (the tiled GEMM needs less).
+// The fragments of x and of one slab of W lie in `fws`, whatever the other workspaces have grown to. The plain
+// rows' workspace is still grown (or refused) as for the tiled GEMM: the same call may be captured next.
+// Returns BRIK_OK with `done` false when `fws` could not be had (the tiled GEMM needs less).
 int gemm_frag(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, const void* sc, const void* mn,
               float* y, int M, int K, int N, bool& done)
 {
     const FragShape s = frag_shape(M, K, N);
     done = false;
-    if (ensure_buf(c, c->ws, c->ws_bytes, s.xbytes) != BRIK_OK) return BRIK_OK;
-    if (!ensure_fws(c, s.wbytes)) return BRIK_OK;
+    long Kp;
+    uint16_t* plain;
+    float* rscale;
+    HIP_TRY_RC(gemm_stage_ws(c, M, K, Kp, plain, rscale));
+    if (!ensure_fws(c, s.xbytes + s.wbytes)) return BRIK_OK;
     done = true;
     c->last_path = BRIK_PATH_TILED;
     c->last_kernel = "gemm_frag";
-    uint16_t* xf = static_cast<uint16_t*>(c->ws);
-    float* rscale = reinterpret_cast<float*>(static_cast<char*>(c->ws) + (size_t)s.RB * s.S * 1024);
-    uint16_t* wf = static_cast<uint16_t*>(c->fws);
+    uint16_t* xf = static_cast<uint16_t*>(c->fws);
+    rscale = reinterpret_cast<float*>(static_cast<char*>(c->fws) + (size_t)s.RB * s.S * 1024);
+    uint16_t* wf = reinterpret_cast<uint16_t*>(static_cast<char*>(c->fws) + s.xbytes);
     int S = (int)s.S;
     for (long cb0 = 0; cb0 < s.CB; cb0 += s.slab) {
         int n0 = (int)(32 * cb0), CB = (int)std::min(s.slab, s.CB - cb0), Ns = (int)std::min<long>(32L * CB, N - n0);
@@ -1922,13 +1922,13 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
     long Kp;
     uint16_t* xh;
     float* rscale;
-    HIP_TRY_RC(gemm_stage_ws(c, M, K, Kp, xh, rscale));
+    int S = (K + 31) / 32 * 2;
+    const size_t xbytes = (size_t)((M + 31) / 32) * S * 1024, hbytes = xbytes + 4 * (size_t)M;   // fragments of x, scales
+    HIP_TRY_RC(gemm_stage_ws(c, M, K, Kp, xh, rscale, nullptr, hbytes));
     if (c->opt_tile == 0) {
         // the f16-weight GEMM over fragments of x (gemm_frag.hip), or the few-row GEMM where it is modelled
-        // faster; the older kernels below serve forced tiles, and a workspace that holds the plain rows but
-        // not whole panels of 32 (it is not grown here: graphs may hold its address)
-        int S = (K + 31) / 32 * 2, ht = 0;
-        const size_t xbytes = (size_t)((M + 31) / 32) * S * 1024;
+        // faster; the older kernels below serve forced tiles
+        int ht = 0;
         double h_us = 0;
         for (int t = 0; t < kNumHalfTiles; ++t) {
             const HalfTile& g = kHalfTiles[t];
@@ -1943,14 +1943,20 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
             const void* none = nullptr;
             return gemm_few(c, F_F16, x, w, none, none, none, y, M, K, N, nullptr);
         }
-        if (xbytes + 4 * (size_t)M <= c->ws_bytes && xbytes < (1ull << 31)) {
-            float* rs = reinterpret_cast<float*>(static_cast<char*>(c->ws) + xbytes);
+        // whole panels of 32 rows may not fit a workspace that holds the plain rows: it is not grown for them
+        // (graphs may hold its address), they go to the workspace that no graph holds. A capture without room
+        // runs the older kernels, which give the same bits (their k order within a sum is the same)
+        char* xw = hbytes <= c->ws_bytes ? static_cast<char*>(c->ws) : nullptr;
+        if (!xw && !c->graph_capturing && ensure_fws(c, hbytes)) xw = static_cast<char*>(c->fws);
+        if (xw && xbytes < (1ull << 31)) {
+            uint16_t* xf = reinterpret_cast<uint16_t*>(xw);
+            float* rs = reinterpret_cast<float*>(xw + xbytes);
             const int rpb = K <= BRIK_FRAG_ROWS8_MAX_K ? 8 : 4;
-            void* pargs[] = {&x, &xh, &rs, &Mi, &Ki, &S};
+            void* pargs[] = {&x, &xf, &rs, &Mi, &Ki, &S};
             HIP_TRY_RC(launch_fn(c, c->fn[K_FRAG_ROWS_F16], (unsigned)((M + rpb - 1) / rpb), 1, 1024, 0, pargs));
             const HalfTile& g = kHalfTiles[ht];
             c->last_kernel = "gemm_h";
-            void* args[] = {&xh, &rs, &w, &y, &Mi, &Ni, &Ki, &S};
+            void* args[] = {&xf, &rs, &w, &y, &Mi, &Ni, &Ki, &S};
             return launch_fn(c, c->gemm_h[ht], gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()), 1, g.threads(), 0, args);
         }
     }

@@ -49,8 +49,6 @@ struct FTile {
                   VM_X0 < 64 && WA <= 15, "tile");
 };
 
-// Wait until at most N LDS operations of this wave are outstanding (they complete in issue order; the
-// loop issues no scalar loads).
 // The fragment of block i at OFF past `base`, blocks STRIDE bytes apart.
 template <int STRIDE, int OFF = 0>
 __device__ __forceinline__ half8_t ds_read_b128_by(uint32_t base, int i)
@@ -59,6 +57,9 @@ __device__ __forceinline__ half8_t ds_read_b128_by(uint32_t base, int i)
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(base), "i"(OFF + STRIDE * i));
     return v;
 }
+
+// Wait until at most N LDS operations of this wave are outstanding (they complete in issue order; the
+// loop issues no scalar loads).
 template <int N>
 __device__ __forceinline__ void lds_wait_n()
 {

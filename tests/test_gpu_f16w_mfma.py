@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from brimkern_amd.capi import Context
 from helpers import Gpu
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +79,40 @@ def test_weights_that_end_their_allocation(gpu, M, K):
     assert N * K * 2 % 65536 == 0
     x, w = data(M, K, N, M * K)
     check(run(gpu, x, w), x, w)
+
+
+@pytest.mark.parametrize("K", [9728, 9736])
+def test_workspace_history(K):
+    """97 rows fit, as plain f16 rows, the workspace that 80 rows leave; whole panels of 32 do not. Such a call
+    runs the same kernel as after a larger one, and recorded there (the workspace may not grow, an older kernel
+    stands in) it gives the same bits."""
+    N = 96
+    x, w = data(400, K, N, 11)
+    with Context(0) as c:
+        gpu = Gpu(c)
+        xb, wb, yb = gpu.up(x), gpu.up(w.view(np.uint16)), gpu.up(np.zeros(400 * N, np.float32))
+
+        def call(M):
+            c.matmul_t_f16w(xb, wb, yb, M, K, N)
+            return c.last_kernel()
+
+        def result():
+            r = c.download(yb, np.uint32, 97 * N)
+            c.h2d(yb, np.zeros(97 * N, np.float32))
+            return r
+
+        assert call(80) == "gemm_h"
+        c.graph_begin()
+        assert call(97) != "gemm_h"
+        g = c.graph_end()
+        g.launch()
+        recorded = result()
+        assert call(97) == "gemm_h"
+        first = result()
+        g.launch()                       # the call before left the workspace where it was
+        assert np.array_equal(result(), recorded) and np.array_equal(first, recorded)
+        g.destroy()
+        assert call(400) == "gemm_h" and call(97) == "gemm_h"
+        assert np.array_equal(result(), first)
+        check(first.view(np.float32).reshape(97, N), x[:97], w)
+        gpu.free()

@@ -33,6 +33,7 @@ def _call(gpu, fmt, xb, planes, yb, M, K, N, tile):
     gpu.ctx.set_option(BRIK_OPT_GEMM_TILE, tile)
     try:
         getattr(gpu.ctx, "matmul_t_" + fmt)(xb, *planes, yb, M, K, N)
+        assert gpu.ctx.last_kernel() == ("gemm" if tile else "gemm_frag")
     finally:
         gpu.ctx.set_option(BRIK_OPT_GEMM_TILE, 0)
     return gpu.ctx.download(yb, np.float32, M * N).reshape(M, N)
@@ -98,9 +99,11 @@ def test_frag_workspaces_and_graphs():
         ctx.matmul_t_q4(xb, *planes, y1, M, K, small)
         g1 = ctx.graph_end()
         ctx.matmul_t_q4(xb, *planes, y2, M, K, N)
+        assert ctx.last_kernel() == "gemm_frag"
         ref = ctx.download(y2, np.float32, M * N)
         ctx.graph_begin()
         ctx.matmul_t_q4(xb, *planes, y3, M, K, N)
+        assert ctx.last_kernel() == "gemm"
         g2 = ctx.graph_end()
         for _ in range(3):
             g1.launch()
@@ -111,4 +114,28 @@ def test_frag_workspaces_and_graphs():
             assert np.array_equal(ctx.download(y2, np.float32, M * N), ref)
         g1.destroy()
         g2.destroy()
+        gpu.free()
+
+
+def test_frag_workspace_history():
+    """Rows whose plain f16 form fits the workspace that fewer rows left, and whose whole panels of 32 would
+    not: the call takes the fragment GEMM all the same, and a graph recorded before it stays valid."""
+    K, N = 17024, 1000
+    with Context(0) as ctx:
+        gpu = Gpu(ctx)
+        t = synth.q3_tensor(12, N, K)
+        planes = gpu.planes("q3", t)
+        x = synth.normal(13, 1025 * K)
+        xb, yb = gpu.up(x), gpu.up(np.zeros(1025 * N, np.float32))
+        _call(gpu, "q3", xb, planes, yb, 1015, K, N, 13)
+        ctx.graph_begin()
+        ctx.matmul_t_q3(xb, *planes, yb, 1025, K, N)
+        g = ctx.graph_end()
+        g.launch()
+        ref = ctx.download(yb, np.float32, 1025 * N).reshape(1025, N)
+        y = _call(gpu, "q3", xb, planes, yb, 1025, K, N, 0)
+        assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+        g.launch()
+        assert np.array_equal(ctx.download(yb, np.uint32, 1025 * N), ref.view(np.uint32).ravel())
+        g.destroy()
         gpu.free()
