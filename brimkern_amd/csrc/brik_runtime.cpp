@@ -252,7 +252,7 @@ struct brik_ctx {
     int opt_tile = 0;      // 0 auto, else 1 + index into kGemmTiles
     int opt_plan_stage = 0;  // plans: 0 auto, 1 in-block staging, 2 staging launch
     int opt_plan_sets = 0;   // plans: 0 auto, else row sets per block
-    int opt_splitk = 0;      // few-row GEMMs: 0 auto, 1 never split-K, 2 split-K whenever it applies
+    int opt_splitk = 0;      // GEMMs of few rows: 0 auto, 1 neither kernel for them, 2 split-K, 3 the few-row one
     int opt_gemv_blocks = 0; // single-matrix GEMV: 0 auto, else grid cap
     void* ws = nullptr;    // GEMM workspace: f16 activation rows, then per-row scales (grow-only)
     size_t ws_bytes = 0;
@@ -676,20 +676,21 @@ size_t few_part_bytes(Fmt f, long rows, int K, int N)
 }
 
 // Whether a dense call takes the few-row GEMM: where its modelled time beats the tiled GEMM's (small_m_path;
-// 10 % and -1.4 us correct what that model gets wrong at short K). It replaces the split-K kernel for every
-// call that would take it: us per call, before -> after: q4 K = 2560, N = 4096, M = 16 14.3 -> 9.3; K = 9728,
+// 10 % and -1.4 us correct what that model gets wrong at short K). It stands in for the split-K kernel on
+// nearly every call that small_m_path gives to that; the rest, of wide matrices and 33 rows or more, where the two
+// are modelled within a few per cent (q4 36 x 3200 x 9728), keep it. Us per call, split-K -> few rows: q4 K = 2560, N = 4096, M = 16 14.3 -> 9.3; K = 9728,
 // N = 2560, M = 16 27.4 -> 12.6, M = 64 34.2 -> 21.4; q8 M = 33 35.4 -> 19.2; K = 896, N = 4864, M = 16 9.8 ->
 // 6.1. The tiled GEMM keeps wide matrices past 32 rows (K = 2560, N = 9728, M = 64: 18.5 against 21.6).
 bool use_few(const brik_ctx* c, Fmt f, long rows, int K, int N, bool fixed)
 {
-    if (rows > kSplitKMaxRows || c->opt_tile > 0 || c->opt_splitk == 1) return false;
+    if (rows > kSplitKMaxRows || c->opt_tile > 0 || c->opt_splitk == 1 || c->opt_splitk == 2) return false;
     // rows and partial tiles have to fit the no-allocation scratch whoever calls (both entry points take
     // the same path), and x one buffer resource
     const size_t part = few_part_bytes(f, rows, K, N);
     if (splitk_part_off(rows, K) + part > BRIK_NOALLOC_SCRATCH_BYTES || (size_t)rows * K >= (1ull << 29) ||
         (part && !fixed && !c->qws))
         return false;
-    if (f == F_F16 || c->opt_splitk == 2) return true;
+    if (f == F_F16 || c->opt_splitk == 3) return true;
     return few_shape(f, rows, K, N).us < 0.9 * tiled_few_us(f, rows, K, N) + 1.4;
 }
 
@@ -1736,7 +1737,7 @@ struct ConvGemm {
 // 32-channel steps a fragment would straddle taps, past BRIK_CONV_GEMM_MAX_TAPS the staging its LDS.
 bool conv_gemm_plan(brik_ctx* c, long Cin, long HW, long Cout, long taps, long P, size_t stage, ConvGemm& g)
 {
-    if (Cin % 32 || taps > BRIK_CONV_GEMM_MAX_TAPS || c->opt_tile > 0) return false;
+    if (Cin % 32 || taps > BRIK_CONV_GEMM_MAX_TAPS || c->opt_tile > 0 || c->opt_splitk == 2) return false;
     const long RB = (Cout + 31) / 32, T = taps * (Cin / 32);
     g.xbytes = ((size_t)HW * Cin * 2 + 255) & ~(size_t)255;
     g.sbytes = ((size_t)HW * 4 + 255) & ~(size_t)255;
@@ -2546,7 +2547,7 @@ int brik_set_option(brik_ctx* c, int key, int value)
         c->opt_plan_stage = value;
         return BRIK_OK;
     case BRIK_OPT_SPLITK:
-        if (value < 0 || value > 2) return fail(c, BRIK_EINVAL, "BRIK_OPT_SPLITK: %d not in 0..2", value);
+        if (value < 0 || value > 3) return fail(c, BRIK_EINVAL, "BRIK_OPT_SPLITK: %d not in 0..3", value);
         c->opt_splitk = value;
         return BRIK_OK;
     case BRIK_OPT_PLAN_SETS:

@@ -369,7 +369,8 @@ int brik_timer_end(brik_ctx *ctx, float *ms);
 #define BRIK_OPT_PLAN_SETS 5     /* grouped GEMV plans created from now on: 0 auto, else row sets per block
                                     (capped by the LDS the lane partials may use) */
 #define BRIK_OPT_SPLITK 6        /* MFMA GEMMs of few rows (expert-grouped, or at most 64 rows): 0 auto,
-                                    1 never use the split-K kernel, 2 use it whenever no tile is forced */
+                                    1 neither kernel for few rows, 2 the split-K kernel whenever no tile is forced,
+                                    3 the few-row kernel for the dense calls of at most 64 rows that it takes */
 #define BRIK_OPT_GEMV_BLOCKS 7   /* single-matrix GEMV launches: 0 auto, else at most this many blocks
                                     (each block then loops over several row sets) */
 int brik_set_option(brik_ctx *ctx, int key, int value);
@@ -381,7 +382,7 @@ int brik_set_option(brik_ctx *ctx, int key, int value);
 #define BRIK_PATH_GEMV 1         /* decode GEMV kernels, x staged in every block */
 #define BRIK_PATH_GEMV_STAGED 2  /* decode GEMV over an x image staged once per call (large M = 1) */
 #define BRIK_PATH_TILED 3        /* MFMA GEMM tiles over staged f16 rows (dense or expert-grouped) */
-#define BRIK_PATH_SPLITK 4       /* few-row split-K MFMA GEMM (partial tiles summed in slice order) */
+#define BRIK_PATH_SPLITK 4       /* few-row MFMA GEMMs: the few-row and the split-K kernels (slices summed in order) */
 int brik_last_path(const brik_ctx *ctx);
 
 /* The product kernel behind it, by the stem of its name without brik_ ("" before any call, or for K = 0):

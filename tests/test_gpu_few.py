@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture()
 def gpu(ctx):
     g = Gpu(ctx)
-    ctx.set_option(BRIK_OPT_SPLITK, 2)
+    ctx.set_option(BRIK_OPT_SPLITK, 3)
     ctx.set_option(BRIK_OPT_PATH, 2)
     yield g
     ctx.set_option(BRIK_OPT_SPLITK, 0)

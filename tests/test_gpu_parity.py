@@ -11,7 +11,7 @@ import pytest
 import oracle as O
 from brimkern_amd import synth, layout
 from brimkern_amd.capi import (BrikError, BRIK_EINVAL, BRIK_EALIGN, BRIK_OPT_PATH, BRIK_OPT_GEMV_VARIANT,
-                               BRIK_GEMV_VARIANTS, BRIK_OPT_GEMM_TILE, BRIK_GEMM_TILES)
+                               BRIK_GEMV_VARIANTS, BRIK_OPT_GEMM_TILE, BRIK_OPT_SPLITK, BRIK_GEMM_TILES)
 from helpers import Gpu, load_golden, normwise_rel, componentwise_ok, moe_oracle_abs, PLANES, REL_TOL
 
 pytestmark = pytest.mark.gpu
@@ -26,6 +26,7 @@ def gpu(ctx):
     ctx.set_option(BRIK_OPT_PATH, 0)
     ctx.set_option(BRIK_OPT_GEMV_VARIANT, 0)
     ctx.set_option(BRIK_OPT_GEMM_TILE, 0)
+    ctx.set_option(BRIK_OPT_SPLITK, 0)
     g.free()
 
 
@@ -183,7 +184,9 @@ def test_gemm_staged_row_scales(gpu, K):
     planes = gpu.planes("q4", t)
     r, den = oracle_mm("q4", x.ravel(), t, M, K, N)
     gpu.ctx.set_option(BRIK_OPT_PATH, 2)
+    gpu.ctx.set_option(BRIK_OPT_SPLITK, 1)
     y = gpu.matmul("q4", x.ravel(), planes, M, K, N)
+    assert gpu.ctx.last_kernel() == "gemm"
     check(y, r, den, REL_TOL)
     assert not np.any(y[3])
 

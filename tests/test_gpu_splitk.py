@@ -1,10 +1,9 @@
 """GPU parity of the split-K few-row GEMM (brik_gemm_sk_<fmt>_k<KSL>) through the C ABI: dense calls of
 few rows and expert-grouped (MoE) calls, against the oracle at the 1e-3 bar (normwise and
 componentwise), over every slice size the runtime picks from (one slice, and several slices whose
-partials the last block of each tile sums), ragged M / N / K, empty experts and experts of more than
-one 32-row tile. The sum over slices runs in slice order whatever order the blocks finish in, so
-repeated calls are bit-identical; the tile counters are left at zero by every call, so calls of other
-shapes in between do not disturb it.
+partials brik_splitk_reduce sums), ragged M / N / K, empty experts and experts of more than one 32-row
+tile. The sum over slices runs in slice order, so repeated calls are bit-identical, also with calls of
+other shapes in between. Every test asserts the kernel that ran.
 """
 import numpy as np
 import pytest
@@ -53,8 +52,9 @@ def test_splitk_dense(gpu, fmt, M, K, N):
     planes = gpu.planes(fmt, t)
     r, den = oracle_mm(fmt, x, t, M)
     y = gpu.matmul(fmt, x, planes, M, K, N)
+    assert gpu.ctx.last_kernel() == "gemm_sk"
     check(y, r, den)
-    # again, after a call of another shape: bit-identical (slice order, counters back at zero)
+    # again, after a call of another shape: bit-identical (slice order)
     t2 = synth.tensor(fmt, 1100, 200, 512)
     gpu.matmul(fmt, synth.normal(1101, 7 * 512), gpu.planes(fmt, t2), 7, 512, 200)
     y2 = gpu.matmul(fmt, x, planes, M, K, N)
@@ -70,10 +70,28 @@ def test_splitk_matches_tiled_kernel(gpu):
     planes = gpu.planes("q4", t)
     r, den = oracle_mm("q4", x, t, M)
     a = gpu.matmul("q4", x, planes, M, K, N)
+    assert gpu.ctx.last_kernel() == "gemm_sk"
     gpu.ctx.set_option(BRIK_OPT_GEMM_TILE, 8)
     b = gpu.matmul("q4", x, planes, M, K, N)
+    assert gpu.ctx.last_kernel() == "gemm"
     check(a, r, den)
     check(b, r, den)
+
+
+@pytest.mark.parametrize("fmt", ["q4", "q8", "q3"])
+def test_splitk_by_default(gpu, fmt):
+    """A call that takes the split-K kernel unasked: its staged rows alone pass the fixed scratch that the few-row
+    kernel's calls have to fit."""
+    M, K, N = 64, 147456, 70
+    gpu.ctx.set_option(BRIK_OPT_SPLITK, 0)
+    gpu.ctx.set_option(BRIK_OPT_PATH, 0)
+    t = synth.tensor(fmt, 1250 + M, N, K)
+    x = synth.normal(1251 + M, M * K)
+    y = gpu.matmul(fmt, x, gpu.planes(fmt, t), M, K, N)
+    assert gpu.ctx.last_kernel() == "gemm_sk"
+    deq = getattr(O, f"dequant_{fmt}")(*[t[k] for k in PLANES[fmt]]).reshape(N, K)
+    w, xd = deq.astype(np.float64).T, x.reshape(M, K).astype(np.float64)
+    check(y, xd @ w, np.abs(xd) @ np.abs(w))
 
 
 @pytest.mark.parametrize("K,N", [(2048, 768), (768, 2048), (1056, 300)])
@@ -90,6 +108,7 @@ def test_splitk_moe(gpu, K, N):
     xb, rb = gpu.up(x), gpu.up(row_off)
     yb = gpu.up(np.full(R * N, np.nan, np.float32))
     gpu.ctx.moe_matmul_t_q4(xb, rb, *planes, yb, E, R, K, N)
+    assert gpu.ctx.last_kernel() == "gemm_sk"
     y = gpu.ctx.download(yb, np.float32, R * N).reshape(R, N)
     r = O.moe_matmul_t_q4(x, row_off, t["nib"], t["sc"], t["mn"], E, K, N)
     deq = O.dequant_q4(t["nib"], t["sc"], t["mn"]).reshape(E, N, K).astype(np.float64)
@@ -106,7 +125,7 @@ def test_splitk_moe(gpu, K, N):
 
 def test_splitk_moe_cfg5_shapes(gpu):
     """The benchmark's MoE layer (256 tokens, top-8 of 64 experts, gate 2048 -> 768, down 768 -> 2048) on
-    the automatic choice, which is the split-K kernel for expert-grouped calls."""
+    the automatic choice, which stays with the tiled kernel for expert-grouped calls."""
     gpu.ctx.set_option(BRIK_OPT_SPLITK, 0)
     T, H, E, F, TOPK = 256, 2048, 64, 768, 8
     rows, row_off = synth.moe_routing(77, T, E, TOPK)
@@ -118,6 +137,7 @@ def test_splitk_moe_cfg5_shapes(gpu):
         xb, rb = gpu.up(x), gpu.up(row_off)
         yb = gpu.up(np.full(R * N, np.nan, np.float32))
         gpu.ctx.moe_matmul_t_q4(xb, rb, *planes, yb, E, R, K, N)
+        assert gpu.ctx.last_kernel() == "gemmg"
         y = gpu.ctx.download(yb, np.float32, R * N)
         r = O.moe_matmul_t_q4(x, row_off, t["nib"], t["sc"], t["mn"], E, K, N)
         assert normwise_rel(y, r) <= REL_TOL

@@ -56,8 +56,9 @@ def check(y, r, den):
 # tiled launch's rows by one wave (K <= 2048) and one block each, and rows read twice
 @pytest.mark.parametrize("fmt", ["q8", "q4", "q3"])
 @pytest.mark.parametrize("M,K,N,splitk,tile", [
-    (6, 544, 33, 0, 0), (12, 1056, 65, 0, 0), (12, 416, 65, 0, 0), (30, 1312, 130, 0, 0), (61, 544, 70, 0, 0),
-    (9, 544, 40, 1, 0), (33, 1312, 40, 1, 0), (33, 2592, 40, 1, 0), (9, 8224, 33, 1, 0), (70, 1312, 64, 0, 13),
+    (6, 544, 33, 3, 0), (12, 1056, 65, 3, 0), (12, 416, 65, 3, 0), (30, 1312, 130, 3, 0), (61, 544, 70, 3, 0),
+    (9, 544, 40, 2, 0), (33, 1312, 40, 2, 0),
+    (9, 544, 40, 0, 8), (33, 1312, 40, 0, 8), (33, 2592, 40, 0, 8), (9, 8224, 33, 0, 8), (70, 1312, 64, 0, 13),
 ])
 def test_matmul_rows(gpu, fmt, M, K, N, splitk, tile):
     t = synth.tensor(fmt, 70 + M, N, K)
@@ -67,6 +68,7 @@ def test_matmul_rows(gpu, fmt, M, K, N, splitk, tile):
     gpu.ctx.set_option(BRIK_OPT_SPLITK, splitk)
     gpu.ctx.set_option(BRIK_OPT_GEMM_TILE, tile)
     check(gpu.matmul(fmt, x.ravel(), gpu.planes(fmt, t), M, K, N), r, den)
+    assert gpu.ctx.last_kernel() == ("gemm" if tile else {2: "gemm_sk", 3: "gemm_few"}[splitk])
 
 
 def test_fragment_rows(gpu):
@@ -75,6 +77,7 @@ def test_fragment_rows(gpu):
     t = synth.tensor("q4", 80, N, K)
     x = rows(M, K, 81)
     y = gpu.matmul("q4", x.ravel(), gpu.planes("q4", t), M, K, N)
+    assert gpu.ctx.last_kernel() == "gemm_frag"
     r, den = O.matmul_t_q4(np.ascontiguousarray(x[:16]).ravel(), t["nib"], t["sc"], t["mn"], 16, K, N, absden=True)
     assert np.isfinite(y).all()
     check(y[:16], r, den)

@@ -1,10 +1,10 @@
 """The no-allocation entry point (brik_matmul_t_q4_noalloc) through the C ABI against the ordinary
 brik_matmul_t_q4 on the same inputs: the same kernels run on the library's fixed per-device scratch
 instead of the context workspaces, so the outputs must be bit-identical. Two calls in a row, the
-second smaller, on each path that uses scratch (the tiled MFMA GEMM's staged f16 rows; the split-K
-GEMM's staged rows and partial tiles; the staged image of a large M = 1 GEMV) and on one that uses
-none, each call's path asserted (brik_last_path); a call needing more than the scratch holds is refused
-before anything runs; and the call records into a graph and replays like the eager call, also after a
+second smaller, on each path that uses scratch (the tiled MFMA GEMM's staged f16 rows; the few-row
+GEMM's partial tiles, behind the room of staged rows; the staged image of a large M = 1 GEMV) and on one
+that uses none, each call's path asserted (brik_last_path); a call needing more than the scratch holds
+is refused before anything runs; and the call records into a graph and replays like the eager call, also after a
 larger eager call has reallocated the context workspace.
 """
 import numpy as np
@@ -41,7 +41,7 @@ def both(gpu, M, K, N, seed):
 
 @pytest.mark.parametrize("first,second,path", [
     ((512, 2560, 1024), (96, 2560, 1024), BRIK_PATH_TILED),       # staged f16 rows in the scratch
-    ((32, 9728, 2560), (24, 2560, 2560), BRIK_PATH_SPLITK),       # staged rows, then the partial tiles
+    ((32, 9728, 2560), (24, 2560, 2560), BRIK_PATH_SPLITK),       # the few-row kernel's partial tiles
     ((1, 2560, 24583), (1, 512, 24577), BRIK_PATH_GEMV_STAGED),   # the staged x image in the scratch
     ((1, 2560, 4096), (1, 1024, 700), BRIK_PATH_GEMV),            # staging in-block: no scratch at all
 ], ids=["gemm", "splitk", "gemv_staged", "gemv"])
