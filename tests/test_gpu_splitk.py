@@ -82,7 +82,7 @@ def test_splitk_matches_tiled_kernel(gpu):
 def test_splitk_by_default(gpu, fmt):
     """A call that takes the split-K kernel unasked: its staged rows alone pass the fixed scratch that the few-row
     kernel's calls have to fit."""
-    M, K, N = 64, 147456, 70
+    M, K, N = 64, 147456, 330
     gpu.ctx.set_option(BRIK_OPT_SPLITK, 0)
     gpu.ctx.set_option(BRIK_OPT_PATH, 0)
     t = synth.tensor(fmt, 1250 + M, N, K)
@@ -90,8 +90,9 @@ def test_splitk_by_default(gpu, fmt):
     y = gpu.matmul(fmt, x, gpu.planes(fmt, t), M, K, N)
     assert gpu.ctx.last_kernel() == "gemm_sk"
     deq = getattr(O, f"dequant_{fmt}")(*[t[k] for k in PLANES[fmt]]).reshape(N, K)
-    w, xd = deq.astype(np.float64).T, x.reshape(M, K).astype(np.float64)
-    check(y, xd @ w, np.abs(xd) @ np.abs(w))
+    cols = np.r_[0:20, N - 20:N]
+    w, xd = deq[cols].astype(np.float64).T, x.reshape(M, K).astype(np.float64)
+    check(y[:, cols], xd @ w, np.abs(xd) @ np.abs(w))
 
 
 @pytest.mark.parametrize("K,N", [(2048, 768), (768, 2048), (1056, 300)])
