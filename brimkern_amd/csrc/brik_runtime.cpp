@@ -638,7 +638,9 @@ int gemm_splitk(brik_ctx* c, Fmt f, const uint16_t* xh, const float* rscale, con
 // K slices over blocks by the modelled time: 4.2 us of launch and ends, `piece_us` per piece of a k wave (x 1.1
 // q8, 1.2 q3; a quarter more per further block on the CU), and with more than one slice 2.7 us for the
 // launch that sums them plus the partial tiles written and read at 2.5 TB/s. Within 10 % at the median of 128
-// measured calls (M 3-64, K 256-9728, N 318-15467).
+// measured calls (M 3-64, K 256-9728, N 318-15467). Slice counts whose partial tiles do not fit the no-allocation
+// scratch behind the staged rows are left out (one slice needs none); not for f16 weights, whose other kernel is
+// the faster one there (64 x 9728 x 8192: 41.8 us against 59.0 with the slices that fit).
 struct FewShape {
     int tile;
     unsigned gx, ks;
@@ -659,7 +661,10 @@ FewShape few_shape(Fmt f, long rows, int K, int N)
         const int n = (int)(((long)s.gx * ks + kCUs - 1) / kCUs);     // blocks on the fullest CU
         const int shared = std::min(n, g.per_cu), rounds = (n + g.per_cu - 1) / g.per_cu;
         double us = 4.2 + rounds * it * u * (1 + 0.25 * (shared - 1));
-        if (ks > 1) us += 2.7 + 8.0 * ks * rows * N / 2.5e6;
+        if (ks > 1) {
+            if (f != F_F16 && splitk_part_off(rows, K) + 4 * (size_t)ks * rows * N > BRIK_NOALLOC_SCRATCH_BYTES) continue;
+            us += 2.7 + 8.0 * ks * rows * N / 2.5e6;
+        }
         if (s.ks == 0 || us < s.us) {
             s.us = us;
             s.ks = (unsigned)ks;
@@ -676,11 +681,12 @@ size_t few_part_bytes(Fmt f, long rows, int K, int N)
 }
 
 // Whether a dense call takes the few-row GEMM: where its modelled time beats the tiled GEMM's (small_m_path;
-// 10 % and -1.4 us correct what that model gets wrong at short K). It stands in for the split-K kernel on
-// nearly every call that small_m_path gives to that; the rest, of wide matrices and 33 rows or more, where the two
-// are modelled within a few per cent (q4 36 x 3200 x 9728), keep it. Us per call, split-K -> few rows: q4 K = 2560, N = 4096, M = 16 14.3 -> 9.3; K = 9728,
-// N = 2560, M = 16 27.4 -> 12.6, M = 64 34.2 -> 21.4; q8 M = 33 35.4 -> 19.2; K = 896, N = 4864, M = 16 9.8 ->
-// 6.1. The tiled GEMM keeps wide matrices past 32 rows (K = 2560, N = 9728, M = 64: 18.5 against 21.6).
+// 10 % and -1.4 us correct what that model gets wrong at short K), and instead of the split-K kernel wherever
+// small_m_path prefers that. Us per call, split-K -> few rows: q4 K = 2560, N = 4096, M = 16 14.3 -> 9.3; K = 9728,
+// N = 2560, M = 16 27.4 -> 12.6, M = 64 34.2 -> 21.4; q8 M = 33 35.4 -> 19.2; K = 896, N = 4864, M = 16 9.8 -> 6.1;
+// wide matrices, where the two are modelled alike: q4 36 x 3200 x 9728 23.1 -> 19.6, q8 40 x 3200 x 12000 30.3 ->
+// 22.3, q3 64 x 4096 x 9728 39.9 -> 26.1. The tiled GEMM keeps other wide matrices past 32 rows (K = 2560, N = 9728,
+// M = 64: 18.5 against 21.6).
 bool use_few(const brik_ctx* c, Fmt f, long rows, int K, int N, bool fixed)
 {
     if (rows > kSplitKMaxRows || c->opt_tile > 0 || c->opt_splitk == 1 || c->opt_splitk == 2) return false;
@@ -691,7 +697,8 @@ bool use_few(const brik_ctx* c, Fmt f, long rows, int K, int N, bool fixed)
         (part && !fixed && !c->qws))
         return false;
     if (f == F_F16 || c->opt_splitk == 3) return true;
-    return few_shape(f, rows, K, N).us < 0.9 * tiled_few_us(f, rows, K, N) + 1.4;
+    return few_shape(f, rows, K, N).us < 0.9 * tiled_few_us(f, rows, K, N) + 1.4 ||
+           small_m_path(f, rows, K, N) == SM_SPLITK;
 }
 
 int gemm_few(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1, const void* sc, const void* mn,

@@ -75,3 +75,20 @@ def test_few_last_rows_and_scales(gpu):
         x = synth.normal(2201 + K, 5 * K)
         y, r, den = run(gpu, "q3", t, x, 5)
         assert np.all(np.abs(y.astype(np.float64) - r) <= REL_TOL * den + 1e-30), (K, N)
+
+
+# wide matrices of 33 rows or more, which the model of the split-K kernel would take, and one whose best slice count
+# would not fit the no-allocation scratch (fewer slices do)
+@pytest.mark.parametrize("fmt,M,K,N", [("q4", 36, 3200, 9728), ("q8", 40, 3200, 12000), ("q3", 64, 4096, 9728),
+                                       ("q4", 64, 9728, 8192)])
+def test_few_in_place_of_splitk(gpu, fmt, M, K, N):
+    gpu.ctx.set_option(BRIK_OPT_SPLITK, 0)
+    gpu.ctx.set_option(BRIK_OPT_PATH, 0)
+    t = synth.tensor(fmt, 2300 + M, N, K)
+    x = synth.normal(2301 + M, M * K)
+    y = gpu.matmul(fmt, x, gpu.planes(fmt, t), M, K, N)
+    assert gpu.ctx.last_kernel() == "gemm_few"
+    deq = getattr(O, f"dequant_{fmt}")(*[t[k] for k in PLANES[fmt]]).reshape(N, K)
+    cols = np.r_[0:40, N - 40:N]
+    w, xd = deq[cols].astype(np.float64).T, x.reshape(M, K).astype(np.float64)
+    assert np.all(np.abs(y[:, cols] - xd @ w) <= REL_TOL * (np.abs(xd) @ np.abs(w)))
