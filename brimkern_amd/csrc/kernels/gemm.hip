@@ -97,14 +97,14 @@ constexpr int XPREP_BCH = 4;
 constexpr int XPREP_WAVE_KP = 2048;
 
 // The power-of-two scale that fits a row of largest magnitude mx into f16: up = 2^(15 - e) multiplies
-// the row, the row's rscale 2^(e - 15) undoes it (zero and non-finite maxima: scale 1). Both stay normal
-// numbers: below 2^-112 the scale stops at 2^126 (2^127 and past it overflow up or make down subnormal), where
-// even the smallest subnormal f32, 2^-149, is still 2 ulp of an f16 subnormal.
+// the row, the row's rscale 2^(e - 15) undoes it (non-finite maxima: scale 1). Both stay normal numbers:
+// below 2^-112, zero included, the scale stops at 2^126 (2^127 and past it overflow up or make down subnormal),
+// where even the smallest subnormal f32, 2^-149, is still 2 ulp of an f16 subnormal.
 __device__ __forceinline__ float xprep_up(float mx, float& down)
 {
     int e = 15;
-    if (mx > 0.f && mx <= 3.4028235e38f) (void)frexpf(mx, &e);    // mx = f * 2^e, f in [0.5, 1)
-    e = max(e, -111);
+    mx = fmaxf(mx, 0x1p-112f);
+    if (mx <= 3.4028235e38f) (void)frexpf(mx, &e);                // mx = f * 2^e, f in [0.5, 1)
     down = ldexpf(1.f, e - 15);
     return ldexpf(1.f, 15 - e);
 }
