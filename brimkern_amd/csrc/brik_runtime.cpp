@@ -144,6 +144,7 @@ constexpr FragTile kFragTiles[] = {{2, 4, 3, 2, 0.29}, {1, 8, 4, 1, 0.165}, {1, 
 constexpr int kNumFragTiles = sizeof(kFragTiles) / sizeof(kFragTiles[0]);
 // dequantized weight panels held at a time: wider matrices run in column slabs of this many bytes
 constexpr size_t kFragSlabBytes = 128u << 20;
+constexpr size_t kConvWeightBytes = 128u << 20;   // most weight fragments of the tap-by-tap convolution
 
 constexpr unsigned kCUs = 256;                 // MI355X compute units
 constexpr long kGemmKPad = 256;                // staged activation rows are padded to this many halves
@@ -267,6 +268,10 @@ struct brik_ctx {
     void* qws = nullptr;   // few-row GEMM: partial tiles (fixed size, so graphs may hold its address)
     void* fws = nullptr;   // fragment GEMM: x panels and the f16 weight panels of one column slab (grow-only)
     size_t fws_bytes = 0;
+    // convolution GEMM: weight fragments (fixed size, taken at the context's first convolution GEMM, so graphs may
+    // hold its address)
+    void* kws = nullptr;
+    bool kws_tried = false;
 
     // pinned staging ring of brik_h2d_async (allocated on first use): uploads in flight as
     // {offset, bytes, event} in issue order; events are recycled through a free list
@@ -1467,6 +1472,7 @@ void brik_destroy(brik_ctx* c)
     if (c->cws) (void)hipFree(c->cws);
     if (c->pws) (void)hipFree(c->pws);
     if (c->fws) (void)hipFree(c->fws);
+    if (c->kws) (void)hipFree(c->kws);
     if (c->qws) (void)hipFree(c->qws);
     if (c->module) (void)hipModuleUnload(c->module);
     delete c;
@@ -1735,13 +1741,18 @@ int brik_quantize_q3(brik_ctx* c, const float* src, uint32_t* lo, uint32_t* hi, 
 struct ConvGemm {
     int tile, sps, ks;
     size_t xbytes, sbytes, wbytes;   // staged pixel rows, their scales, weight fragments
+    bool fits;                       // the fragments lie behind the pixel rows, else in kws
 };
 
 // Whether the call can run it: taps of whole 32-channel steps, the pixel rows inside the workspace the im2col
-// rows (`stage` bytes) need anyway, the weight fragments behind them or, where no graph would come to hold
-// its address, in the slab of the fragment GEMM. It then replaces im2col staging and the tiled GEMM at every
-// size: 1.2 to 3 times as fast on 22 shapes of 8-75 x 8-92 pixels, 32-608 channels, 1 x 1 to 5 x 5. Without whole
-// 32-channel steps a fragment would straddle taps, past BRIK_CONV_GEMM_MAX_TAPS the staging its LDS.
+// rows (`stage` bytes) need anyway, the weight fragments behind them or in the context's fixed buffer. All of that
+// depends on the shape alone, so a recorded call runs the kernels of the eager one. It then replaces im2col
+// staging and the tiled GEMM: 1.2 to 3 times as fast on 22 shapes of 8-75 x 8-92 pixels, 32-608 channels, 1 x 1
+// to 5 x 5, and with the fragments in the fixed buffer (640-2560 channels, 8-16 x 8-16 pixels, 3 x 3) 1.6 to 2.6
+// times: q4 1280 x 16 x 16, 1280 channels 80.2 -> 37.4 us, 2560 channels in 142.7 -> 58.6. The pixel rows of a
+// strided call hold every input pixel, the im2col rows only those it reads: a 1 x 1 kernel of stride 2 keeps
+// im2col. Without whole 32-channel steps a fragment would straddle taps, past BRIK_CONV_GEMM_MAX_TAPS the staging
+// its LDS.
 bool conv_gemm_plan(brik_ctx* c, long Cin, long HW, long Cout, long taps, long P, size_t stage, ConvGemm& g)
 {
     if (Cin % 32 || taps > BRIK_CONV_GEMM_MAX_TAPS || c->opt_tile > 0 || c->opt_splitk == 2) return false;
@@ -1749,8 +1760,8 @@ bool conv_gemm_plan(brik_ctx* c, long Cin, long HW, long Cout, long taps, long P
     g.xbytes = ((size_t)HW * Cin * 2 + 255) & ~(size_t)255;
     g.sbytes = ((size_t)HW * 4 + 255) & ~(size_t)255;
     g.wbytes = (size_t)RB * T * 2048;
-    if (g.xbytes + g.sbytes > stage || g.wbytes > kFragSlabBytes) return false;
-    if (g.xbytes + g.sbytes + g.wbytes > stage && c->graph_capturing) return false;
+    g.fits = g.xbytes + g.sbytes + g.wbytes <= stage;
+    if (g.xbytes + g.sbytes > stage || (!g.fits && (!c->kws || g.wbytes > kConvWeightBytes))) return false;
     double best = 0;
     for (int t = 0; t < kNumConvTiles; ++t) {
         const HalfTile& h = kConvTiles[t];
@@ -1775,8 +1786,8 @@ bool conv_gemm_plan(brik_ctx* c, long Cin, long HW, long Cout, long taps, long P
     return true;
 }
 
-// Convolution with a quantized weight: an MFMA GEMM, tap by tap (conv_gemm_plan) or over im2col rows, when the weight rows are whole groups
-// (K = Cin kh kw a multiple of 32) and the shape is large enough for the GEMM tiles, else the direct
+// Convolution with a quantized weight: an MFMA GEMM, tap by tap (conv_gemm_plan) or over im2col rows, when the
+// weight rows are whole groups (K = Cin kh kw a multiple of 32) and the shape is large enough for the GEMM tiles, else the direct
 // kernel. Option BRIK_OPT_PATH 1 forces the direct kernel, 2 the GEMM (when K % 32 == 0).
 static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const void* p0, const uint16_t* sc,
                   const uint16_t* mn, const float* bias, float* out, int Cin, int H, int W, int Cout, int kh, int kw,
@@ -1830,6 +1841,14 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
     // the GEMM writes out itself ([Cout, pixels] plus the bias) unless the split-K kernel runs it
     const bool fused = !use_splitk(c, f, rows, Kint, Cout, 0);
     HIP_TRY_RC(ensure_buf(c, c->cws, c->cws_bytes, (fused ? 0 : yt_bytes) + (size_t)H * W * 4));
+    // (a capture past this point follows an eager call that grew cws, and so the attempt below)
+    if (!c->kws_tried && !c->graph_capturing) {
+        c->kws_tried = true;
+        if (hipMalloc(&c->kws, kConvWeightBytes) != hipSuccess) {
+            (void)hipGetLastError();
+            c->kws = nullptr;
+        }
+    }
     float* yt = static_cast<float*>(c->cws);
     float* cmax = reinterpret_cast<float*>(static_cast<unsigned char*>(c->cws) + (fused ? 0 : yt_bytes));
     int Kpi = (int)Kp, HW = H * W;
@@ -1838,27 +1857,23 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
         char* const wsp = static_cast<char*>(c->ws);
         uint16_t* xt = reinterpret_cast<uint16_t*>(wsp);
         float* xs = reinterpret_cast<float*>(wsp + cg.xbytes);
-        uint16_t* wf = reinterpret_cast<uint16_t*>(wsp + cg.xbytes + cg.sbytes);
-        const bool room = cg.xbytes + cg.sbytes + cg.wbytes <= c->ws_bytes;
-        if (room || ensure_fws(c, cg.wbytes)) {
-            if (!room) wf = static_cast<uint16_t*>(c->fws);
-            c->last_path = BRIK_PATH_TILED;
-            c->last_kernel = "gemm_conv";
-            int taps = kh * kw, xblocks = (HW + 15) / 16, P = rows;
-            void* pargs[] = {&inp, &xt, &xs, &p0, &sc, &mn, &wf, &Ci, &HW, &Co, &taps, &xblocks};
-            HIP_TRY_RC(launch_fn(c, c->conv_prep[f == F_Q4],
-                                 (unsigned)xblocks + (unsigned)((Cout + 31) / 32) * (unsigned)(Cin / 32), 1, 1024, 0, pargs));
-            const HalfTile& t = kConvTiles[cg.tile];
-            float* part = static_cast<float*>(c->qws);
-            void* args[] = {&wf, &xt, &xs, &bias, &out, &part, &Ci, &Hi, &Wi, &Co, &kwi, &taps, &si, &pi, &OWi, &P, &cg.sps};
-            HIP_TRY_RC(launch_fn(c, c->gemm_conv[cg.tile], gemm_tiles(Cout, t.bm()) * gemm_tiles(rows, t.bn()),
-                                 (unsigned)cg.ks, t.threads(), 0, args));
-            if (cg.ks == 1) return BRIK_OK;
-            size_t n = (size_t)Cout * rows;
-            void* rargs[] = {&part, &out, &n, &cg.ks};
-            const size_t blocks = (n + 255) / 256;
-            return launch(c, K_SPLITK_REDUCE, (unsigned)(blocks < 2048 ? blocks : 2048), 1, 256, 0, rargs);
-        }
+        uint16_t* wf = reinterpret_cast<uint16_t*>(cg.fits ? wsp + cg.xbytes + cg.sbytes : static_cast<char*>(c->kws));
+        c->last_path = BRIK_PATH_TILED;
+        c->last_kernel = "gemm_conv";
+        int taps = kh * kw, xblocks = (HW + 15) / 16, P = rows;
+        void* pargs[] = {&inp, &xt, &xs, &p0, &sc, &mn, &wf, &Ci, &HW, &Co, &taps, &xblocks};
+        HIP_TRY_RC(launch_fn(c, c->conv_prep[f == F_Q4],
+                             (unsigned)xblocks + (unsigned)((Cout + 31) / 32) * (unsigned)(Cin / 32), 1, 1024, 0, pargs));
+        const HalfTile& t = kConvTiles[cg.tile];
+        float* part = static_cast<float*>(c->qws);
+        void* args[] = {&wf, &xt, &xs, &bias, &out, &part, &Ci, &Hi, &Wi, &Co, &kwi, &taps, &si, &pi, &OWi, &P, &cg.sps};
+        HIP_TRY_RC(launch_fn(c, c->gemm_conv[cg.tile], gemm_tiles(Cout, t.bm()) * gemm_tiles(rows, t.bn()),
+                             (unsigned)cg.ks, t.threads(), 0, args));
+        if (cg.ks == 1) return BRIK_OK;
+        size_t n = (size_t)Cout * rows;
+        void* rargs[] = {&part, &out, &n, &cg.ks};
+        const size_t blocks = (n + 255) / 256;
+        return launch(c, K_SPLITK_REDUCE, (unsigned)(blocks < 2048 ? blocks : 2048), 1, 256, 0, rargs);
     }
     {
         void* args[] = {&inp, &cmax, &Ci, &HW};

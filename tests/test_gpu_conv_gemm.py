@@ -10,8 +10,9 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from brimkern_amd.capi import BRIK_OPT_PATH
-from helpers import Gpu
+from brimkern_amd import layout
+from brimkern_amd.capi import BRIK_OPT_PATH, Context
+from helpers import Gpu, PLANES
 from test_gpu_conv import quantized, run
 
 pytestmark = pytest.mark.gpu
@@ -26,7 +27,8 @@ def gpu(ctx):
 
 
 SHAPES = [
-    (32, 8, 8, 1, 1, 1, 1, 0),         # one step in all, one channel
+    (32, 8, 8, 16, 1, 1, 1, 0),        # one step in all
+    (512, 8, 8, 1, 1, 1, 1, 0),        # one output channel
     (32, 9, 11, 33, 3, 3, 1, 1),       # one step per tap
     (64, 17, 15, 65, 3, 3, 2, 1),      # stride 2, every tile ragged
     (96, 12, 13, 16, 5, 5, 1, 2),      # 25 taps, sliced sum
@@ -49,6 +51,7 @@ def test_conv_gemm(gpu, fmt, bias, shape):
     x = (rng.standard_normal((Cin, H, W)) * 2.0 ** rng.integers(-20, 20, (1, H, W))).astype(np.float32)
     b = rng.standard_normal(Cout).astype(np.float32) if bias else None
     y = run(gpu, fmt, x, blob, w.size, b, shape, 2).astype(np.float64)
+    assert gpu.ctx.last_kernel() == "gemm_conv"
     wt = torch.from_numpy(np.asarray(deq, dtype=np.float64).reshape(Cout, Cin, kh, kw))
     xt = torch.from_numpy(x.astype(np.float64))[None]
     ref = F.conv2d(xt, wt, stride=st, padding=pd)[0].numpy()
@@ -58,3 +61,47 @@ def test_conv_gemm(gpu, fmt, bias, shape):
         den = den + np.abs(b)[:, None, None]
     tol = 2.0 ** -10 + Cin * kh * kw * 2.0 ** -24
     assert np.all(np.abs(y - ref) <= tol * den)
+
+
+# weight fragments behind the pixel rows, and past the im2col rows' size (a buffer of their own)
+@pytest.mark.parametrize("shape", [(32, 40, 40, 40, 3, 3, 1, 1), (256, 8, 8, 200, 3, 3, 1, 1), (512, 8, 8, 64, 1, 1, 1, 0)],
+                         ids=["behind", "apart", "apart1x1"])
+def test_recorded_conv_runs_the_eager_kernel(shape):
+    """A convolution recorded before it ever ran eagerly, on workspaces that another one left, gives the bits of
+    the eager call, also replayed after larger eager calls."""
+    Cin, H, W, Cout, kh, kw, st, pd = shape
+    rng = np.random.default_rng(sum(shape))
+    blob, _ = quantized("q4", rng.standard_normal(Cout * Cin * kh * kw).astype(np.float32))
+    n, pixels = Cout * Cin * kh * kw, H * W
+    with Context(0) as c:
+        gpu = Gpu(c)
+        buf, xb = gpu.up(blob), gpu.up(rng.standard_normal(Cin * H * W).astype(np.float32))
+        planes = [buf.offset(layout.plane_offsets("q4", n)[p][0]) for p in PLANES["q4"]]
+        y = gpu.up(np.zeros(Cout * pixels, np.float32))
+
+        def other(side):
+            b, _ = quantized("q4", rng.standard_normal(32 * 32 * 9).astype(np.float32))
+            run(gpu, "q4", rng.standard_normal((32, side, side)).astype(np.float32), b, 32 * 32 * 9, None,
+                (32, side, side, 32, 3, 3, 1, 1), 0)
+
+        def bits():
+            r = c.download(y, np.uint32, Cout * pixels)
+            c.h2d(y, np.zeros(Cout * pixels, np.float32))
+            return r
+
+        other(64)                               # 2.1 MB of im2col rows
+        c.graph_begin()
+        c.conv2d("q4", xb, planes, None, y, *shape)
+        assert c.last_kernel() == "gemm_conv"
+        g = c.graph_end()
+        g.launch()
+        recorded = bits()
+        c.conv2d("q4", xb, planes, None, y, *shape)
+        assert c.last_kernel() == "gemm_conv"
+        assert np.array_equal(bits(), recorded) and recorded.any()
+        for _ in range(3):
+            other(40)
+            g.launch()
+            assert np.array_equal(bits(), recorded)
+        g.destroy()
+        gpu.free()
