@@ -1741,7 +1741,8 @@ int brik_quantize_q3(brik_ctx* c, const float* src, uint32_t* lo, uint32_t* hi, 
 struct ConvGemm {
     int tile, sps, ks;
     size_t xbytes, sbytes, wbytes;   // staged pixel rows, their scales, weight fragments
-    bool fits;                       // the fragments lie behind the pixel rows, else in kws
+    bool fits;                       // the fragments lie behind the pixel rows (at woff), else in kws
+    size_t woff() const { return (xbytes + sbytes + 255) & ~(size_t)255; }
 };
 
 // Whether the call can run it: taps of whole 32-channel steps, the pixel rows inside the workspace the im2col
@@ -1757,10 +1758,10 @@ bool conv_gemm_plan(brik_ctx* c, long Cin, long HW, long Cout, long taps, long P
 {
     if (Cin % 32 || taps > BRIK_CONV_GEMM_MAX_TAPS || c->opt_tile > 0 || c->opt_splitk == 2) return false;
     const long RB = (Cout + 31) / 32, T = taps * (Cin / 32);
-    g.xbytes = ((size_t)HW * Cin * 2 + 255) & ~(size_t)255;
-    g.sbytes = ((size_t)HW * 4 + 255) & ~(size_t)255;
+    g.xbytes = (size_t)HW * Cin * 2;
+    g.sbytes = (size_t)HW * 4;
     g.wbytes = (size_t)RB * T * 2048;
-    g.fits = g.xbytes + g.sbytes + g.wbytes <= stage;
+    g.fits = g.woff() + g.wbytes <= stage;
     if (g.xbytes + g.sbytes > stage || (!g.fits && (!c->kws || g.wbytes > kConvWeightBytes))) return false;
     double best = 0;
     for (int t = 0; t < kNumConvTiles; ++t) {
@@ -1857,7 +1858,7 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
         char* const wsp = static_cast<char*>(c->ws);
         uint16_t* xt = reinterpret_cast<uint16_t*>(wsp);
         float* xs = reinterpret_cast<float*>(wsp + cg.xbytes);
-        uint16_t* wf = reinterpret_cast<uint16_t*>(cg.fits ? wsp + cg.xbytes + cg.sbytes : static_cast<char*>(c->kws));
+        uint16_t* wf = reinterpret_cast<uint16_t*>(cg.fits ? wsp + cg.woff() : static_cast<char*>(c->kws));
         c->last_path = BRIK_PATH_TILED;
         c->last_kernel = "gemm_conv";
         int taps = kh * kw, xblocks = (HW + 15) / 16, P = rows;

@@ -29,6 +29,7 @@ def gpu(ctx):
 SHAPES = [
     (32, 8, 8, 16, 1, 1, 1, 0),        # one step in all
     (512, 8, 8, 1, 1, 1, 1, 0),        # one output channel
+    (512, 9, 9, 40, 1, 1, 1, 0),       # pixel rows that just fit the im2col rows' room
     (32, 9, 11, 33, 3, 3, 1, 1),       # one step per tap
     (64, 17, 15, 65, 3, 3, 2, 1),      # stride 2, every tile ragged
     (96, 12, 13, 16, 5, 5, 1, 2),      # 25 taps, sliced sum
