@@ -1,6 +1,7 @@
-"""Build-time check of the GEMM kernels' inline-asm LDS reads (brik_gemm*, gemm.hip).
+"""Build-time check of the GEMM kernels' inline-asm LDS reads (brik_gemm*: gemm.hip, gemm_frag.hip,
+conv_gemm.hip).
 
-The multiply loop issues its LDS reads as inline asm (gemm.hip: ds_read_b128 / ds_read_u16, then
+The multiply loops issue their LDS reads as inline asm (ds_read_b128 / ds_read_u16 / ds_read_b32, then
 lds_wait and tie), so the compiler does not know that their destination registers are written
 asynchronously. Correctness then rests on register allocation: no instruction may read or write a
 destination register of such a read before an `s_waitcnt lgkmcnt` has retired it.
@@ -11,7 +12,7 @@ instructions (targets from their 16-bit word offsets; a conditional branch also 
 unconditional one and s_endpgm do not) and propagates the registers still pending from an LDS read
 forward to a fixed point, so a read issued at the bottom of a loop is still pending at the loop's head
 on the back edge. The disassembly does not tell the asm reads from the compiler's own, so every
-ds_read_b128 / ds_read_u16 is tracked. A pending register carries its age, the number of LGKM-counted
+read of those three forms is tracked. A pending register carries its age, the number of LGKM-counted
 operations (LDS, scalar memory) issued after its read, and at a join the smaller age of the paths:
 LDS operations complete in issue order, so `s_waitcnt lgkmcnt(N)` retires the reads of age N or more,
 unless a scalar memory load may be in flight (those complete out of order, and then only lgkmcnt(0)
@@ -28,7 +29,7 @@ import sys
 
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 OBJDUMP = os.path.join(ROCM, "llvm", "bin", "llvm-objdump")
-ASM_READS = ("ds_read_b128", "ds_read_u16")
+ASM_READS = ("ds_read_b128", "ds_read_b32", "ds_read_u16")
 MAX_AGE = 16          # lgkmcnt holds at most 15 on gfx9: an older read is retired by any lgkmcnt wait
 
 
@@ -41,8 +42,9 @@ def _regs(op: str) -> set:
 
 
 def _checked(fn: str) -> bool:
-    """The tiled GEMM kernels (gemm_body): brik_gemm_<fmt>_<tile> and brik_gemmg_q4_<tile>. The split-K
-    kernels and the f16-weight LDS-tiled kernel read LDS the ordinary way (compiler-tracked waits)."""
+    """The GEMM kernels: brik_gemm_<fmt>_<tile>, brik_gemmg_q4_<tile>, brik_gemm_frag_*, brik_gemm_h_*,
+    brik_gemm_conv_* (and brik_gemm_few_*, which waits the ordinary way). The split-K kernels and the
+    f16-weight LDS-tiled kernel read LDS the ordinary way (compiler-tracked waits)."""
     return fn.startswith(("brik_gemm_", "brik_gemmg_")) and not fn.startswith(("brik_gemm_sk_", "brik_gemm_f16w"))
 
 

@@ -130,3 +130,23 @@ def test_join_keeps_the_younger_age():
     ])
     bad = check(text)
     assert len(bad) == 1 and "v[7]" in bad[0]
+
+
+def test_every_asm_read_form_is_tracked():
+    """Each form of LDS read that the kernels issue as inline asm, by its own register width."""
+    for read, reg in (("ds_read_b128 v[2:5], v44", 5), ("ds_read_b32 v5, v44 offset:128", 5), ("ds_read_u16 v5, v44", 5)):
+        text = HEAD.format("brik_gemm_conv_22_1x1") + body([read, f"v_mul_f32_e32 v9, v{reg}, v8", "s_waitcnt lgkmcnt(0)"])
+        bad = check(text)
+        assert len(bad) == 1 and f"v[{reg}]" in bad[0], read
+
+
+def test_tracked_forms_are_those_of_the_sources():
+    """Every LDS read written as inline asm in the kernel sources is of a tracked form."""
+    import os
+    import re
+    from brimkern_amd import check_lds_reads as C
+    root = os.path.join(os.path.dirname(os.path.abspath(C.__file__)), "csrc", "kernels")
+    forms = set()
+    for f in os.listdir(root):
+        forms |= set(re.findall(r'asm[^;]*"(ds_read\w*)', open(os.path.join(root, f)).read()))
+    assert forms and forms <= set(C.ASM_READS), forms
