@@ -436,6 +436,7 @@ int ensure_buf(brik_ctx* c, void*& buf, size_t& have, size_t bytes)
     if (c->graph_capturing)
         return fail(c, BRIK_EINVAL, "a workspace would grow during graph capture: run the same calls once "
                                     "before brik_graph_begin");
+    HIP_TRY(c, hipSetDevice(c->device));           // the calling thread may have another device current
     if (buf) {
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         HIP_TRY(c, hipFree(buf));
@@ -789,6 +790,7 @@ int gemm_run(brik_ctx* c, Fmt f, const uint16_t* xh, const float* rscale, const 
 bool ensure_fws(brik_ctx* c, size_t bytes)
 {
     if (c->fws_bytes >= bytes) return true;
+    if (hipSetDevice(c->device) != hipSuccess) return false;
     if (c->fws) {
         if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
         (void)hipFree(c->fws);
@@ -1845,6 +1847,7 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
     // (a capture past this point follows an eager call that grew cws, and so the attempt below)
     if (!c->kws_tried && !c->graph_capturing) {
         c->kws_tried = true;
+        HIP_TRY(c, hipSetDevice(c->device));
         if (hipMalloc(&c->kws, kConvWeightBytes) != hipSuccess) {
             (void)hipGetLastError();
             c->kws = nullptr;
