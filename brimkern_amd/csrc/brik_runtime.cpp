@@ -96,17 +96,20 @@ constexpr GemmTile kGemmTiles[] = {{128, 2, 4, 1}, {128, 1, 4, 1}, {128, 3, 4, 1
                                    {64, 1, 4, 3},  {32, 1, 8, 2},  {64, 1, 8, 2}};
 constexpr int kNumGemmTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
-// f16-weight GEMM tiles (gemm_frag.hip, brik_gemm_h_*), as kFragTiles: 192 x 256, 256 x 128, 128 x 128, 64 x 64.
-// Fastest of 14 tiles at (M, K, N) = (4096, 9728, 2560) 188 us, (512, 2560, 9728) 34.9, (777, 2560, 4096) 24.6 and
-// (256, 2560, 9728) 23.3, (128, 2560, 2560) 11.6.
-struct HalfTile {
+// Block tiles of the GEMMs over fragments (gemm_frag.hip, conv_gemm.hip): WR x WC waves of WA x WB 32 x 32 blocks
+// each. `slice_us`: time of a 16-k slice per round of CUs, measured on the product alone.
+struct FragTile {
     int wr, wc, wa, wb;
     double slice_us;
     int bm() const { return 32 * wr * wa; }
     int bn() const { return 32 * wc * wb; }
     unsigned threads() const { return 64u * (unsigned)(wr * wc); }
 };
-constexpr HalfTile kHalfTiles[] = {{2, 4, 3, 2, 0.32}, {4, 2, 2, 2, 0.21}, {4, 2, 1, 2, 0.135}, {2, 2, 1, 1, 0.055}};
+
+// f16-weight GEMM (brik_gemm_h_*): 192 x 256, 256 x 128, 128 x 128, 64 x 64. Fastest of 14 tiles at (M, K, N) =
+// (4096, 9728, 2560) 188 us, (512, 2560, 9728) 34.9, (777, 2560, 4096) 24.6 and (256, 2560, 9728) 23.3,
+// (128, 2560, 2560) 11.6.
+constexpr FragTile kHalfTiles[] = {{2, 4, 3, 2, 0.32}, {4, 2, 2, 2, 0.21}, {4, 2, 1, 2, 0.135}, {2, 2, 1, 1, 0.055}};
 constexpr int kNumHalfTiles = sizeof(kHalfTiles) / sizeof(kHalfTiles[0]);
 
 // Few-row GEMM tiles (gemm_few.hip): up to `rows` rows, CW x KW waves, 32 CW columns per block, in the order
@@ -123,23 +126,14 @@ constexpr FewTile kFewTiles[] = {{8, 1, 4, 2.0, 3}, {16, 1, 4, 2.1, 2}, {16, 2, 
 constexpr int kNumFewTiles = sizeof(kFewTiles) / sizeof(kFewTiles[0]);
 constexpr int kFewK = 256;                     // k of one piece (FEW_K)
 
-// Convolution GEMM tiles (conv_gemm.hip), as kHalfTiles (rows: output channels, columns: pixels); the time of a
-// slice with a block on every CU.
-constexpr HalfTile kConvTiles[] = {{2, 2, 1, 1, 0.1}, {4, 2, 1, 2, 0.17}};
+// Convolution GEMM (rows: output channels, columns: pixels); the time of a slice with a block on every CU.
+constexpr FragTile kConvTiles[] = {{2, 2, 1, 1, 0.1}, {4, 2, 1, 2, 0.17}};
 constexpr int kNumConvTiles = sizeof(kConvTiles) / sizeof(kConvTiles[0]);
 
-// Fragment GEMM tiles (gemm_frag.hip): WR x WC waves of WA x WB 32 x 32 blocks each, in the order of
-// BRIK_FRAG_TILES: 192 x 256, 128 x 256, 128 x 128, 64 x 128. `slice_us`: time of a 16-k slice per round of
-// CUs, measured on the product alone. Swept at (M, K, N) = (4096, 9728, 2560), (2048 and 1024, 2560, 9728),
-// (777, 2560, 4096), (512, 2560, 9728), (4096, 2560, 320): each of the four is the fastest of 18 tiles
-// (64-256 rows, 128-256 columns, 4 and 8 waves) on one of them, 174, 98, 53, 21.7, 29.9 and 12.4 us.
-struct FragTile {
-    int wr, wc, wa, wb;
-    double slice_us;
-    int bm() const { return 32 * wr * wa; }
-    int bn() const { return 32 * wc * wb; }
-    unsigned threads() const { return 64u * (unsigned)(wr * wc); }
-};
+// Fragment GEMM, in the order of BRIK_FRAG_TILES: 192 x 256, 128 x 256, 128 x 128, 64 x 128. Swept at (M, K, N) =
+// (4096, 9728, 2560), (2048 and 1024, 2560, 9728), (777, 2560, 4096), (512, 2560, 9728), (4096, 2560, 320): each of
+// the four is the fastest of 18 tiles (64-256 rows, 128-256 columns, 4 and 8 waves) on one of them, 174, 98, 53,
+// 21.7, 29.9 and 12.4 us.
 constexpr FragTile kFragTiles[] = {{2, 4, 3, 2, 0.29}, {1, 8, 4, 1, 0.165}, {1, 4, 4, 1, 0.115}, {1, 4, 2, 1, 0.068}};
 constexpr int kNumFragTiles = sizeof(kFragTiles) / sizeof(kFragTiles[0]);
 // dequantized weight panels held at a time: wider matrices run in column slabs of this many bytes
@@ -826,19 +820,21 @@ FragShape frag_shape(long M, long K, long N)
     return s;
 }
 
-// The tile of fewest rounds of CUs x time per slice.
-int frag_tile(long M, long N)
+// The tile of fewest rounds of CUs x time per slice, and that product.
+template <int T>
+int frag_tile(const FragTile (&tiles)[T], long M, long N, double* slice_us = nullptr)
 {
     int best = 0;
     double best_us = 0;
-    for (int t = 0; t < kNumFragTiles; ++t) {
-        const FragTile& g = kFragTiles[t];
+    for (int t = 0; t < T; ++t) {
+        const FragTile& g = tiles[t];
         const double us = g.slice_us * std::ceil((double)gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()) / kCUs);
         if (t == 0 || us < best_us) {
             best = t;
             best_us = us;
         }
     }
+    if (slice_us) *slice_us = best_us;
     return best;
 }
 
@@ -859,7 +855,7 @@ bool use_frag(brik_ctx* c, Fmt f, long M, long K, long N)
     constexpr double kSliceUs[kNumFragTiles] = {0.28, 0.178, 0.086, 0.056};   // per round, as fitted
     const double mk = (double)M * K, nk = (double)N * K, mn = (double)M * N;
     const double wb = f == F_Q4 ? 0.625 : f == F_Q8 ? 1.0625 : 0.5;
-    const int ft = frag_tile(M, std::min<long>(N, 32 * s.slab));
+    const int ft = frag_tile(kFragTiles, M, std::min<long>(N, 32 * s.slab));
     const double slabs = std::ceil((double)s.CB / s.slab);
     const double frounds = std::ceil((double)gemm_tiles(M, kFragTiles[ft].bm()) * gemm_tiles(N, kFragTiles[ft].bn()) / kCUs);
     const double frag_us = 10.2 * slabs + (6 * mk + (2 + wb) * nk + 4 * mn) / 6.2e6 + s.S * frounds * kSliceUs[ft];
@@ -900,7 +896,7 @@ int gemm_frag(brik_ctx* c, Fmt f, const float* x, const void* p0, const void* p1
         const unsigned wblocks = (unsigned)(((long)CB * (S / 8) + 15) / 16);
         void* pargs[] = {&x, &xf, &rscale, &p0, &p1, &sc, &mn, &wf, &M, &K, &n0, &N, &CB, &S, &xblocks};
         HIP_TRY_RC(launch_fn(c, c->frag_prep[fmt_index(f)], (unsigned)xblocks + wblocks, 1, 1024, 0, pargs));
-        const int t = frag_tile(M, Ns);
+        const int t = frag_tile(kFragTiles, M, Ns);
         const FragTile& g = kFragTiles[t];
         float* ys = y + n0;
         void* args[] = {&xf, &rscale, &wf, &ys, &M, &Ns, &N, &S};
@@ -1393,7 +1389,7 @@ int brik_create(int device, brik_ctx** out)
     }
     for (int t = 0; t < kNumHalfTiles; ++t) {
         char name[64];
-        const HalfTile& g = kHalfTiles[t];
+        const FragTile& g = kHalfTiles[t];
         snprintf(name, sizeof name, "brik_gemm_h_%d%d_%dx%d", g.wr, g.wc, g.wa, g.wb);
         if (hipModuleGetFunction(&c->gemm_h[t], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
     }
@@ -1409,7 +1405,7 @@ int brik_create(int device, brik_ctx** out)
             return bail(BRIK_EMODULE);
     for (int t = 0; t < kNumConvTiles; ++t) {
         char name[64];
-        const HalfTile& g = kConvTiles[t];
+        const FragTile& g = kConvTiles[t];
         snprintf(name, sizeof name, "brik_gemm_conv_%d%d_%dx%d", g.wr, g.wc, g.wa, g.wb);
         if (hipModuleGetFunction(&c->gemm_conv[t], c->module, name) != hipSuccess) return bail(BRIK_EMODULE);
     }
@@ -1767,7 +1763,7 @@ bool conv_gemm_plan(brik_ctx* c, long Cin, long HW, long Cout, long taps, long P
     if (g.xbytes + g.sbytes > stage || (!g.fits && (!c->kws || g.wbytes > kConvWeightBytes))) return false;
     double best = 0;
     for (int t = 0; t < kNumConvTiles; ++t) {
-        const HalfTile& h = kConvTiles[t];
+        const FragTile& h = kConvTiles[t];
         const long tiles = (long)gemm_tiles(Cout, h.bm()) * gemm_tiles(P, h.bn());
         for (long ks = 1; ks <= 16 && ks <= T; ++ks) {
             const long sps = (T + ks - 1) / ks;
@@ -1868,7 +1864,7 @@ static int conv2d(brik_ctx* c, Fmt f, const char* who, const float* inp, const v
         void* pargs[] = {&inp, &xt, &xs, &p0, &sc, &mn, &wf, &Ci, &HW, &Co, &taps, &xblocks};
         HIP_TRY_RC(launch_fn(c, c->conv_prep[f == F_Q4],
                              (unsigned)xblocks + (unsigned)((Cout + 31) / 32) * (unsigned)(Cin / 32), 1, 1024, 0, pargs));
-        const HalfTile& t = kConvTiles[cg.tile];
+        const FragTile& t = kConvTiles[cg.tile];
         float* part = static_cast<float*>(c->qws);
         void* args[] = {&wf, &xt, &xs, &bias, &out, &part, &Ci, &Hi, &Wi, &Co, &kwi, &taps, &si, &pi, &OWi, &P, &cg.sps};
         HIP_TRY_RC(launch_fn(c, c->gemm_conv[cg.tile], gemm_tiles(Cout, t.bm()) * gemm_tiles(rows, t.bn()),
@@ -1955,16 +1951,8 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
     if (c->opt_tile == 0) {
         // the f16-weight GEMM over fragments of x (gemm_frag.hip), or the few-row GEMM where it is modelled
         // faster; the older kernels below serve forced tiles
-        int ht = 0;
-        double h_us = 0;
-        for (int t = 0; t < kNumHalfTiles; ++t) {
-            const HalfTile& g = kHalfTiles[t];
-            const double us = g.slice_us * std::ceil((double)gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()) / kCUs);
-            if (t == 0 || us < h_us) {
-                ht = t;
-                h_us = us;
-            }
-        }
+        double h_us;
+        const int ht = frag_tile(kHalfTiles, M, N, &h_us);
         h_us = 9.0 + h_us * S;
         if (M <= kSplitKMaxRows && use_few(c, F_F16, M, K, N, false) && few_shape(F_F16, M, K, N).us < h_us) {
             const void* none = nullptr;
@@ -1981,7 +1969,7 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
             const int rpb = K <= BRIK_FRAG_ROWS8_MAX_K ? 8 : 4;
             void* pargs[] = {&x, &xf, &rs, &Mi, &Ki, &S};
             HIP_TRY_RC(launch_fn(c, c->fn[K_FRAG_ROWS_F16], (unsigned)((M + rpb - 1) / rpb), 1, 1024, 0, pargs));
-            const HalfTile& g = kHalfTiles[ht];
+            const FragTile& g = kHalfTiles[ht];
             c->last_kernel = "gemm_h";
             void* args[] = {&xf, &rs, &w, &y, &Mi, &Ni, &Ki, &S};
             return launch_fn(c, c->gemm_h[ht], gemm_tiles(M, g.bm()) * gemm_tiles(N, g.bn()), 1, g.threads(), 0, args);
