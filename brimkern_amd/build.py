@@ -37,6 +37,13 @@ SANITIZE_BIN = os.path.join(ROOT, "tests", "native", "host_sanitize")
 HIP_DEVICE_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast",
                     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
+# Load address of the code object's .text. Left to the linker it follows the metadata, so every kernel added
+# anywhere moves the decode kernels, which come first in the code, and with them a decoder layer's time: its four
+# launches start 40 to 70 KB of code each, a pass over cold instruction caches. The same code, a Qwen3-4B q4 layer
+# in us: 27.87-27.94 at 14 of 32 addresses, 27.95-28.03 at 13, 28.08-28.17 at 5 (0x61600, where the metadata
+# had put it, among these); 27.90 here.
+TEXT_ADDR = 0x50000
+
 
 def _run(cmd, verbose):
     if verbose:
@@ -49,7 +56,7 @@ def build_hsaco(verbose=False):
     src = os.path.join(CSRC, "kernels", "brik_kernels.hip")
     tmp = HSACO + ".tmp"
     _run([os.path.join(ROCM, "bin", "hipcc"), "--genco", "--no-gpu-bundle-output", *HIP_DEVICE_FLAGS,
-          "-o", tmp, src], verbose)
+          "-Xoffload-linker", f"--section-start=.text={TEXT_ADDR:#x}", "-o", tmp, src], verbose)
     os.replace(tmp, HSACO)
     return HSACO
 
