@@ -7,7 +7,8 @@
 // [Cout, OH, OW] f32, OH = (H + 2 pad - kh) / s + 1 (likewise OW).
 //
 // Three paths (chosen by the host):
-//   * tap by tap (conv_gemm.hip), from 64 output pixels, when Cin is a multiple of 32 and kh kw at most 25;
+//   * tap by tap (conv_gemm.hip), from 64 output pixels, when Cin is a multiple of 32 and kh kw at most 25 (strided
+//     1 x 1 kernels aside);
 //   * implicit GEMM, for the others whose K = Cin kh kw is a multiple of 32 (then the groups of a weight row are
 //     exactly the matmul's, W[Cout, K]): brik_xprep_im2col_f16 stages the im2col rows of the input
 //     (one per output pixel, K taps) as scaled f16 rows, the way brik_xprep_f16 stages matmul

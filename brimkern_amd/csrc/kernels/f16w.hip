@@ -8,7 +8,8 @@
 //   * brik_gemm_f16w (M > 1, K % 8 == 0): x staged by brik_xprep_f16 (row-scaled f16, the k order
 //     [0 4 1 5 2 6 3 7] within each 8), a 64 x 128 block tile per 4 waves, K steps of 32 through LDS,
 //     v_mfma_f32_32x32x16_f16 with f32 accumulation; W is permuted into the same k order when it is
-//     staged, so A and B contract over matching k.
+//     staged, so A and B contract over matching k. It serves K % 32 != 0 with a forced tile, and captures whose
+//     workspace has no room for the fragments of the GEMM that replaced it (gemm_frag.hip, the same bits).
 #include "common.h"
 
 namespace {
