@@ -237,11 +237,11 @@ def gemv_layer_set(ctx, steps, warmup, layers, settle_s, graph_replay=True):
 
 
 def small_m_rows(ctx, small_m, key, tb, count, one):
-    """``one(i, M)`` at M in SMALL_M on each path (auto, GEMV, tiled, split-K), graph-replayed."""
+    """``one(i, M)`` at M in SMALL_M on each path (auto, GEMV, tiled, split-K, few rows), graph-replayed."""
     for M in SMALL_M:
         row = {}
         for label, path, sk in (("auto", PATH_AUTO, 0), ("gemv", PATH_GEMV, 0), ("tiled", PATH_GEMM, 1),
-                                ("splitk", PATH_GEMM, 2)):
+                                ("splitk", PATH_GEMM, 2), ("few", PATH_GEMM, 3)):
             ctx.set_option(BRIK_OPT_PATH, path)
             ctx.set_option(BRIK_OPT_SPLITK, sk)
             try:
@@ -794,7 +794,7 @@ def main():
     extra = {"per_matrix_single_launch": single, "f3_decode_layers_fused_qwen3_4b": fused,
              "small_m_qwen3_4b": dict(small_m, note="matmul_t_q4 at M rows per call (the reference's "
                                       "matmul_t_q4_tiled range 2 <= M < 16): the routed path (auto), the GEMV "
-                                      "re-streaming W per row, the tiled MFMA GEMM and the split-K MFMA GEMM, "
+                                      "re-streaming W per row, the tiled, the split-K and the few-row MFMA GEMM, "
                                       "graph-replayed; weight_GBps = W bytes (read once) / auto time")}
     if not args.no_extra:
         log("bench: q8 / q3 small-M")
