@@ -1954,16 +1954,20 @@ int brik_matmul_t_f16w(brik_ctx* c, const float* x, const uint16_t* w, float* y,
         double h_us;
         const int ht = frag_tile(kHalfTiles, M, N, &h_us);
         h_us = 9.0 + h_us * S;
-        if (M <= kSplitKMaxRows && use_few(c, F_F16, M, K, N, false) && few_shape(F_F16, M, K, N).us < h_us) {
+        if (M <= kSplitKMaxRows && use_few(c, F_F16, M, K, N, false) &&
+            (c->opt_splitk == 3 || few_shape(F_F16, M, K, N).us < h_us)) {
             const void* none = nullptr;
             return gemm_few(c, F_F16, x, w, none, none, none, y, M, K, N, nullptr);
         }
         // whole panels of 32 rows may not fit a workspace that holds the plain rows: it is not grown for them
         // (graphs may hold its address), they go to the workspace that no graph holds. A capture without room
-        // runs the older kernels, which give the same bits (their k order within a sum is the same)
-        char* xw = hbytes <= c->ws_bytes ? static_cast<char*>(c->ws) : nullptr;
-        if (!xw && !c->graph_capturing && ensure_fws(c, hbytes)) xw = static_cast<char*>(c->fws);
-        if (xw && xbytes < (1ull << 31)) {
+        // runs the older kernels, which give the same bits (each of their MFMAs sums the same 16 k)
+        char* xw = nullptr;                                         // the panels: one buffer resource
+        if (xbytes < (1ull << 31)) {
+            if (hbytes <= c->ws_bytes) xw = static_cast<char*>(c->ws);
+            else if (!c->graph_capturing && ensure_fws(c, hbytes)) xw = static_cast<char*>(c->fws);
+        }
+        if (xw) {
             uint16_t* xf = reinterpret_cast<uint16_t*>(xw);
             float* rs = reinterpret_cast<float*>(xw + xbytes);
             const int rpb = K <= BRIK_FRAG_ROWS8_MAX_K ? 8 : 4;

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from brimkern_amd.capi import Context
+from brimkern_amd.capi import BRIK_OPT_SPLITK, Context
 from helpers import Gpu
 
 pytestmark = pytest.mark.gpu
@@ -18,6 +18,7 @@ pytestmark = pytest.mark.gpu
 def gpu(ctx):
     g = Gpu(ctx)
     yield g
+    ctx.set_option(BRIK_OPT_SPLITK, 0)
     g.free()
 
 
@@ -48,6 +49,7 @@ def check(y, x, w):
 def test_h_tiles(gpu, M, K, N):
     x, w = data(M, K, N, M + K)
     y = run(gpu, x, w)
+    assert gpu.ctx.last_kernel() == "gemm_h"
     check(y, x, w)
     assert np.array_equal(y.view(np.uint32), run(gpu, x, w).view(np.uint32))
 
@@ -56,17 +58,21 @@ def test_h_tiles(gpu, M, K, N):
                                    (32, 1304, 257), (24, 5152, 65), (33, 24, 513), (64, 544, 127), (47, 3104, 130)])
 def test_few_f16(gpu, M, K, N):
     x, w = data(M, K, N, M + K + 1)
+    gpu.ctx.set_option(BRIK_OPT_SPLITK, 3)
     check(run(gpu, x, w), x, w)
+    assert gpu.ctx.last_kernel() == "gemm_few"
 
 
-@pytest.mark.parametrize("M", [5, 40, 200])
+@pytest.mark.parametrize("M,kernel", [(5, "gemm_few"), (40, "gemm_few"), (40, "gemm_h"), (200, "gemm_h")])
 @pytest.mark.parametrize("K", [40, 64, 72, 88])
-def test_infinite_weight_stays_in_its_row(gpu, M, K):
+def test_infinite_weight_stays_in_its_row(gpu, M, K, kernel):
     N = 70
+    gpu.ctx.set_option(BRIK_OPT_SPLITK, 3 if kernel == "gemm_few" else 1)
     x, w = data(M, K, N, 7)
     x = np.abs(x) + np.float32(0.5)
     w[7, 0] = w[69, K - 1] = np.float16(np.inf)
     y = run(gpu, x, w)
+    assert gpu.ctx.last_kernel() == kernel
     cols = [n for n in range(N) if n not in (7, 69)]
     assert np.isposinf(y[:, [7, 69]]).all() and np.isfinite(y[:, cols]).all()
     check(y[:, cols], x, np.ascontiguousarray(w[cols]))
@@ -78,7 +84,9 @@ def test_weights_that_end_their_allocation(gpu, M, K):
     N = 4096
     assert N * K * 2 % 65536 == 0
     x, w = data(M, K, N, M * K)
+    gpu.ctx.set_option(BRIK_OPT_SPLITK, 1)
     check(run(gpu, x, w), x, w)
+    assert gpu.ctx.last_kernel() == "gemm_h"
 
 
 @pytest.mark.parametrize("K", [9728, 9736])

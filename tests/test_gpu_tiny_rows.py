@@ -83,16 +83,19 @@ def test_fragment_rows(gpu):
     check(y[:16], r, den)
 
 
-@pytest.mark.parametrize("M,K,N,tile", [(7, 544, 33, 0), (30, 1312, 130, 0), (200, 1312, 129, 0), (100, 6176, 65, 0),
-                                        (40, 544, 64, 5)])
-def test_f16_rows(gpu, M, K, N, tile):
+@pytest.mark.parametrize("M,K,N,splitk,tile,kernel", [
+    (7, 544, 33, 3, 0, "gemm_few"), (30, 1312, 130, 3, 0, "gemm_few"), (200, 1312, 129, 0, 0, "gemm_h"),
+    (100, 6176, 65, 0, 0, "gemm_h"), (40, 544, 64, 0, 5, "gemm_f16")])
+def test_f16_rows(gpu, M, K, N, splitk, tile, kernel):
     rng = np.random.default_rng(M + K)
     w = (rng.standard_normal((N, K)) * 0.05).astype(np.float16).view(np.uint16)
     x = rows(M, K, 90 + M)
     r, den = O.matmul_t_f16w(x.ravel(), w.ravel(), M, K, N)
+    gpu.ctx.set_option(BRIK_OPT_SPLITK, splitk)
     gpu.ctx.set_option(BRIK_OPT_GEMM_TILE, tile)
     yb = gpu.up(np.full(M * N, np.nan, np.float32))
     gpu.ctx.matmul_t_f16w(gpu.up(x), gpu.up(w), yb, M, K, N)
+    assert gpu.ctx.last_kernel() == kernel
     check(gpu.ctx.download(yb, np.float32, M * N).reshape(M, N), r.reshape(M, N), den.reshape(M, N))
 
 
@@ -113,6 +116,7 @@ def test_conv_pixels(gpu, fmt, shape, tile):
     x[0, 10, 2] = np.float32(2.0 ** -149)
     gpu.ctx.set_option(BRIK_OPT_GEMM_TILE, tile)
     y = run_conv(gpu, fmt, x, blob, w.size, None, shape, 2)
+    assert gpu.ctx.last_kernel() == ("gemm" if tile or Cin % 32 else "gemm_conv")
     wt = torch.from_numpy(np.asarray(deq, dtype=np.float64).reshape(Cout, Cin, kh, kw))
     xt = torch.from_numpy(x.astype(np.float64))[None]
     check(y, F.conv2d(xt, wt, stride=st, padding=pd)[0].numpy(),
